@@ -8,7 +8,9 @@ assembly of every k_gemm_tile instantiation and fails if any instruction
 reads or writes the destination register of an LDS read that no wait has
 retired yet: lgkmcnt(0) retires every read, and the compiler's own
 lgkmcnt(n) retires all but the n youngest LDS operations when no scalar load
-is in flight (LDS operations complete in order).
+is in flight (LDS operations complete in order).  Reads in flight are followed
+along the branches, not in text order: the compiler places blocks of the
+epilogue between blocks of the main loop.
 
     python3 check_lds_asm.py k_gemm.s
 """
@@ -24,46 +26,88 @@ def regset(tok):
     return {tok} if m else set()
 
 
+MAX_QUEUE = 64     # operations remembered per path (more than a wait can name)
+
+
+def blocks_of(body):
+    """Basic blocks [(label, [instructions])] in text order."""
+    out = [(None, [])]
+    for ln in body.split("\n"):
+        t = ln.split(";")[0].strip()
+        m = re.match(r"(\.LBB\w+):", t)
+        if m:
+            out.append((m.group(1), []))
+            continue
+        if not t or t.startswith(".") or t.endswith(":"):
+            continue
+        out[-1][1].append(t)
+        if re.match(r"s_c?branch|s_endpgm|s_setpc", t):
+            out.append((None, []))
+    return out
+
+
+def run_block(instrs, queue, report):
+    """The lgkm operations in flight after the block, oldest first: (destination
+    registers, is scalar memory).  LDS operations complete in order, so a wait
+    lgkmcnt(n) retires all but the n youngest; scalar loads complete out of
+    order, so with one in flight only lgkmcnt(0) retires anything."""
+    queue = list(queue)
+    for t in instrs:
+        ops = [x for x in re.split(r"[ ,]+", t) if x]
+        if ops[0].startswith("ds_"):
+            dst = regset(ops[1]) if ops[0].startswith(("ds_read", "ds_bpermute", "ds_permute",
+                                                       "ds_swizzle")) else set()
+            queue.append((frozenset(dst), False))
+            queue = queue[-MAX_QUEUE:]
+            continue
+        if ops[0].startswith(("s_load", "s_buffer_load")):
+            queue.append((frozenset(), True))
+            queue = queue[-MAX_QUEUE:]
+            continue
+        if ops[0] == "s_waitcnt":
+            m = re.search(r"lgkmcnt\((\d+)\)", t)
+            if m:
+                n = int(m.group(1))
+                if n == 0:
+                    queue = []
+                elif not any(s for _, s in queue):
+                    queue = queue[-n:] if n < len(queue) else queue
+            continue
+        pending = set().union(*(d for d, _ in queue)) if queue else set()
+        if pending:
+            used = set()
+            for o in ops[1:]:
+                used |= regset(o)
+            if used & pending:
+                report(t)
+    return tuple(queue)
+
+
 def check(asm_text):
     bad = []
     names = re.findall(r"^(_Z11k_gemm_tile\S*):", asm_text, re.M)
     for name in names:
-        a = asm_text.index(name + ":")
+        a = asm_text.index(name + ":") + len(name) + 1
         b = asm_text.index(".Lfunc_end", a)
-        # lgkm operations in flight, oldest first: (destination registers, is
-        # scalar memory).  LDS operations complete in order, so a wait
-        # lgkmcnt(n) retires all but the n youngest; scalar loads complete out
-        # of order, so with one in flight only lgkmcnt(0) retires anything.
-        queue = []
-        for ln in asm_text[a:b].split("\n"):
-            t = ln.split(";")[0].strip()
-            if not t or t.startswith("."):
+        blocks = blocks_of(asm_text[a:b])
+        at = {lab: i for i, (lab, _) in enumerate(blocks) if lab}
+        seen = [set() for _ in blocks]
+        found = set()
+        work = [(0, ())]
+        while work:
+            i, queue = work.pop()
+            if queue in seen[i]:
                 continue
-            ops = [x for x in re.split(r"[ ,]+", t) if x]
-            if ops[0].startswith("ds_"):
-                dst = regset(ops[1]) if ops[0].startswith(("ds_read", "ds_bpermute", "ds_permute",
-                                                           "ds_swizzle")) else set()
-                queue.append((dst, False))
-                continue
-            if ops[0].startswith(("s_load", "s_buffer_load")):
-                queue.append((set(), True))
-                continue
-            if ops[0] == "s_waitcnt":
-                m = re.search(r"lgkmcnt\((\d+)\)", t)
-                if m:
-                    n = int(m.group(1))
-                    if n == 0:
-                        queue = []
-                    elif not any(s for _, s in queue):
-                        queue = queue[-n:] if n < len(queue) else queue
-                continue
-            pending = set().union(*(d for d, _ in queue)) if queue else set()
-            if pending:
-                used = set()
-                for o in ops[1:]:
-                    used |= regset(o)
-                if used & pending:
-                    bad.append((name, t))
+            seen[i].add(queue)
+            instrs = blocks[i][1]
+            after = run_block(instrs, queue, lambda t, i=i: found.add((i, t)))
+            last = instrs[-1] if instrs else ""
+            m = re.match(r"s_c?branch\w*\s+(\.LBB\w+)", last)
+            if m:
+                work.append((at[m.group(1)], after))
+            if not re.match(r"s_branch|s_endpgm|s_setpc", last) and i + 1 < len(blocks):
+                work.append((i + 1, after))
+        bad += [(name, t) for _, t in sorted(found)]
     return names, bad
 
 

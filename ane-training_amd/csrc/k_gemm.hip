@@ -26,12 +26,13 @@
  * accumulator i holds C[8*(i/4) + 4*(l/32) + i%4][l%32].
  *
  * Kernels:
- *   k_gemm_tile    work-group tile BM x BN: 64 x 64 for most shapes (four waves
- *                  2 x 2), 256 x 128 for the largest (eight waves 4 x 2), 128 x 128
- *                  (eight waves) K-split in 2 for long-K narrow GEMMs of 1024+
- *                  rows, 64 x 64 also for decode-row classifiers, 32 x 64 for up to
- *                  32 rows (two waves), 32 x 32 (one wave) for decode-row gate
- *                  GEMMs of few tiles; K streamed by direct global->LDS loads into a ring of
+ *   k_gemm_tile    work-group tile BM x BN: 64 x 64 and 64 x 128 (four waves
+ *                  2 x 2), 128 x 128 and 256 x 128 (eight waves 4 x 2), the
+ *                  prefill choice by pick_tile; 128 x 128 K-split in 2 for long-K
+ *                  narrow GEMMs of 1024+ rows; 64 x 64 also for decode-row
+ *                  classifiers, 32 x 64 for up to 32 rows (two waves), 32 x 32
+ *                  (one wave) for decode-row gate GEMMs of few tiles; K streamed
+ *                  by direct global->LDS loads into a ring of
  *                  64-wide stages (3 deep for prefill, 4 for decode rows, 6 for
  *                  32-row gate tiles); XCD-aware tile order; an optional K-split
  *                  over blockIdx.y (fp32 partials, summed by the kernel that
@@ -418,28 +419,22 @@ struct QkvItem {
     float2 c, sn;
 };
 
-/* Position and slot of this thread's items of round `round` (item k: tile row
- * (tid + k*GT) / (BN/4), columns 4 * ((tid + k*GT) % (BN/4)) ..). */
-template <int BM, int BN, int NI>
-__device__ __forceinline__ void qkv_item_rows(QkvItem (&it)[NI], int round, int m0, const EpiArgs &e)
+/* Tile row of row r (0..63) of round q of the QKV epilogue: a round takes the
+ * 32-row tiles i = q / (WVM/2) of the wave rows 2h and 2h + 1, h = q % (WVM/2). */
+template <int BM, int WVM>
+__device__ __forceinline__ int qkv_round_row(int q, int r)
 {
-    constexpr int WM = BM / 2, C4 = BN / 4;
-#pragma unroll
-    for (int k = 0; k < NI; k++) {
-        const int r = (threadIdx.x + k * GT) / C4;
-        const int row = min(m0 + (r >> 5) * WM + round * 32 + (r & 31), e.M - 1);
-        it[k].p = e.pos[row];
-        it[k].sl = e.slot[row];
-    }
+    constexpr int HV = WVM / 2, WM = BM / WVM;
+    return (2 * (q % HV) + (r >> 5)) * WM + (q / HV) * 32 + (r & 31);
 }
 
 /* The items' rotations (clamped indices: the loads stay unconditional). */
-template <int BN, int NI>
+template <int BN, int NT, int NI>
 __device__ __forceinline__ void qkv_item_rope(QkvItem (&it)[NI], int n0, const EpiArgs &e)
 {
 #pragma unroll
     for (int k = 0; k < NI; k++) {
-        const int n = n0 + 4 * ((threadIdx.x + k * GT) % (BN / 4));
+        const int n = n0 + 4 * ((threadIdx.x + k * NT) % (BN / 4));
         const bool rot = n < e.NQ + e.NKV;
         const int nn = n < e.NQ ? n : n - e.NQ;
         const int ti = rot ? it[k].p * (e.hd >> 1) + ((nn & (e.hd - 1)) >> 1) : 0;
@@ -449,60 +444,69 @@ __device__ __forceinline__ void qkv_item_rope(QkvItem (&it)[NI], int n0, const E
 }
 
 /* QKV epilogue of a BM x BN work-group tile through LDS: in rounds of 64 rows
- * (row tile i of both wave rows), the fp32 products are staged in LDS, then
- * each thread takes 4 consecutive columns of a row (two RoPE pairs,
+ * (one 32-row tile of each of two wave rows), the fp32 products are staged in
+ * LDS, then each thread takes 4 consecutive columns of a row (two RoPE pairs,
  * forward.h:55-70): q columns go to q [M, NQ] with one 16-byte store, k and v
  * columns to the cache at (slot[row], pos[row]) with one 16- or 8-byte store.
  * pre: positions and slots of round 0's items, loaded before the main loop
- * (TM = 1), or NULL.  b0, b1:
- * LDS of at least 64 * BN floats each, no longer read by any wave's main loop. */
-template <int BM, int BN, int TM, int TN, int NI>
+ * (one round), or NULL; with several rounds they are loaded for all of them
+ * first, and a round's rotations while the one before it is stored, so that
+ * the rounds do not each wait for two dependent loads.  b0, b1: LDS of at
+ * least 64 * BN floats each, no longer read by any wave's main loop. */
+template <int BM, int BN, int TM, int TN, int WVM, int NI>
 __device__ __forceinline__ void qkv_tile_lds(const f32x16 (&acc)[TM][TN], float *b0, float *b1,
                                              int m0, int n0, int wm, int wn, const EpiArgs &e,
                                              const QkvItem (*pre)[NI], bool own = true)
 {
-    constexpr int WM = BM / 2, WN = BN / 2, C4 = BN / 4;
-    static_assert(NI * GT == 64 * C4, "items per thread");
+    constexpr int WN = BN / 2, C4 = BN / 4, HV = WVM / 2, R = TM * HV, NT = 128 * WVM;
+    static_assert(NI * NT == 64 * C4, "items per thread");
     const int lane = threadIdx.x & 63;
+    QkvItem its[R][NI];   /* (only round q's and q + 1's rotations are live at once) */
+    if (own) {   /* the waves of other K groups (own false) only keep the barriers */
+#pragma unroll
+        for (int q = 0; q < R; q++)
+#pragma unroll
+            for (int k = 0; k < NI; k++) {
+                if (q == 0 && pre) {
+                    its[q][k] = (*pre)[k];
+                } else {
+                    const int row = min(m0 + qkv_round_row<BM, WVM>(q, (threadIdx.x + k * NT) / C4), e.M - 1);
+                    its[q][k].p = e.pos[row];
+                    its[q][k].sl = e.slot[row];
+                }
+            }
+    }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-        float *buf = (i & 1) ? b1 : b0;
-        /* buf row wm*32 + r holds tile row m0 + wm*WM + i*32 + r; the waves
-         * of other K groups (own false) only keep the barriers */
-        QkvItem its[NI];
-        if (own) {
+    for (int q = 0; q < R; q++) {
+        float *buf = (q & 1) ? b1 : b0;
+        if (own && (wm >> 1) == q % HV) {   /* buf row r: tile row qkv_round_row(q, r) */
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
                 for (int k = 0; k < 16; k++) {
-                    const int r = wm * 32 + 8 * (k >> 2) + 4 * (lane >> 5) + (k & 3);
-                    buf[r * BN + wn * WN + j * 32 + (lane & 31)] = acc[i][j][k];
+                    const int r = (wm & 1) * 32 + 8 * (k >> 2) + 4 * (lane >> 5) + (k & 3);
+                    buf[r * BN + wn * WN + j * 32 + (lane & 31)] = acc[q / HV][j][k];
                 }
-            if (i == 0 && pre) {
-#pragma unroll
-                for (int k = 0; k < NI; k++) its[k] = (*pre)[k];
-            } else {
-                qkv_item_rows<BM, BN, NI>(its, i, m0, e);
-            }
-            qkv_item_rope<BN, NI>(its, n0, e);
         }
+        if (own && q == 0) qkv_item_rope<BN, NT, NI>(its[0], n0, e);
+        if (own && q + 1 < R) qkv_item_rope<BN, NT, NI>(its[q + 1 < R ? q + 1 : q], n0, e);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < NI; k++) {
             if (!own) break;
-            const int idx = threadIdx.x + k * GT, r = idx / C4, c4 = idx % C4;
-            const int row = m0 + (r >> 5) * WM + i * 32 + (r & 31);
+            const int idx = threadIdx.x + k * NT, r = idx / C4, c4 = idx % C4;
+            const int row = m0 + qkv_round_row<BM, WVM>(q, r);
             const int n = n0 + 4 * c4;
             if (row >= e.M || n >= e.N) continue;
             const float4 v = *(const float4 *)(buf + r * BN + 4 * c4);
-            const int p = its[k].p;
+            const int p = its[q][k].p;
             const bool isq = n < e.NQ, rot = n < e.NQ + e.NKV;
             const int nn = isq ? n : (rot ? n - e.NQ : n - e.NQ - e.NKV);
             const int d = nn & (e.hd - 1);
             float o[4] = {v.x, v.y, v.z, v.w};
             if (rot) {
-                const float2 c = its[k].c, sn = its[k].sn;
+                const float2 c = its[q][k].c, sn = its[q][k].sn;
                 o[0] = fmaf(v.x, c.x, -(v.y * sn.x));   /* forward.h:64 */
                 o[1] = fmaf(v.x, sn.x, v.y * c.x);      /* forward.h:65 */
                 o[2] = fmaf(v.z, c.y, -(v.w * sn.y));
@@ -512,7 +516,7 @@ __device__ __forceinline__ void qkv_tile_lds(const f32x16 (&acc)[TM][TN], float 
                 *(float4 *)(e.q + (size_t)row * e.NQ + n) = make_float4(o[0], o[1], o[2], o[3]);
             } else {
                 const size_t off =
-                    (((size_t)its[k].sl * e.Hkv + (nn >> e.lghd)) * e.max_seq + p) * e.hd + d;
+                    (((size_t)its[q][k].sl * e.Hkv + (nn >> e.lghd)) * e.max_seq + p) * e.hd + d;
                 void *dst = rot ? e.kc : e.vc;
                 if (e.kv_f32)
                     *(float4 *)((float *)dst + off) = make_float4(o[0], o[1], o[2], o[3]);
@@ -538,8 +542,8 @@ __global__ void __launch_bounds__(64 * WVM * WVN * KG) k_gemm_tile(const u16 *__
     constexpr int STAGE = ROWS * 64;            /* halves per stage (128 B per row) */
     constexpr int LDW = ROWS / 8 / NWV;         /* load instructions per wave per stage */
     static_assert(TM >= 1 && TN >= 1 && LDW >= 1 && ROWS % (8 * NWV) == 0, "tile shape");
-    /* the LDS-staged QKV epilogue is written for four waves */
-    static_assert((WVM == 2 && WVN == 2) || E != EPI_QKV, "wave layout");
+    /* the LDS-staged QKV epilogue takes pairs of wave rows of two waves */
+    static_assert(((WVM == 2 || WVM == 4) && WVN == 2) || E != EPI_QKV, "wave layout");
     static_assert(WVN == 1 || WVN == 2, "one or two waves along N");
     static_assert(NS >= 3 && NS <= 8 && LDW * (NS - 2) <= 63, "ring depth (vmcnt holds 63)");
     static_assert(KG == 1 || ((E == EPI_GATE || E == EPI_STORE || E == EPI_QKV) && !RS),
@@ -680,9 +684,10 @@ __global__ void __launch_bounds__(64 * WVM * WVN * KG) k_gemm_tile(const u16 *__
     /* positions and slots of a one-round tile's QKV epilogue, loaded first so
      * that they arrive during the main loop */
     constexpr bool QKV_LDS = E == EPI_QKV && 64 * BN * 2 <= STAGE;
-    constexpr int QNI = 64 * BN / 4 / GT;
+    constexpr int QNI = 64 * BN / 4 / (64 * NWV);
+    constexpr bool QPRE = QKV_LDS && TM == 1 && WVM == 2;
     QkvItem qpre[QKV_LDS ? QNI : 1];
-    if constexpr (QKV_LDS && TM == 1) {
+    if constexpr (QPRE) {
 #pragma unroll
         for (int k = 0; k < QNI; k++) {
             if (KG > 1 && kg > 0) break;
@@ -692,19 +697,22 @@ __global__ void __launch_bounds__(64 * WVM * WVN * KG) k_gemm_tile(const u16 *__
             qpre[k].sl = e.slot[row];
         }
     }
-    /* the residual a one-tile wave adds (RESID, RESNORM) and the gain
-     * (RESNORM), loaded before the ring so that they arrive during the main
-     * loop instead of after it */
-    constexpr bool XPRE = (E == EPI_RESID || E == EPI_RESNORM) && TM * TN == 1;
-    float xpre[XPRE ? 17 : 1];
+    /* the residual that a wave of one or two tiles adds (RESID, RESNORM) and
+     * the gain (RESNORM), loaded before the ring so that they arrive during
+     * the main loop instead of after it */
+    constexpr bool XPRE = (E == EPI_RESID || E == EPI_RESNORM) && TM * TN <= 2;
+    float xpre[XPRE ? TM * TN : 1][XPRE ? 17 : 1];
     if constexpr (XPRE) {
-        const int n = n0 + wn * WN + (lane & 31);
-        const int rb = m0 + wm * WM + 4 * (lane >> 5);
-        if constexpr (E == EPI_RESNORM) xpre[16] = n < N ? e.gain[n] : 0.f;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int r = rb + 8 * (i >> 2) + (i & 3);
-            xpre[i] = r < M && n < N ? e.out[(size_t)r * e.ldc + n] : 0.f;
+        for (int t = 0; t < TM * TN; t++) {
+            const int n = n0 + wn * WN + (t % TN) * 32 + (lane & 31);
+            const int rb = m0 + wm * WM + (t / TN) * 32 + 4 * (lane >> 5);
+            if constexpr (E == EPI_RESNORM) xpre[t][16] = n < N ? e.gain[n] : 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int r = rb + 8 * (i >> 2) + (i & 3);
+                xpre[t][i] = r < M && n < N ? e.out[(size_t)r * e.ldc + n] : 0.f;
+            }
         }
     }
     /* Row scale after a RESNORM GEMM (RS, e.rs_ss set): thread r < BM loads
@@ -796,8 +804,8 @@ __global__ void __launch_bounds__(64 * WVM * WVN * KG) k_gemm_tile(const u16 *__
         return;
     }
     if constexpr (QKV_LDS) {
-        qkv_tile_lds<BM, BN, TM, TN, QNI>(acc, (float *)lds0, (float *)lds1, m0, n0, wm, wn, e,
-                                          TM == 1 ? &qpre : nullptr, kg == 0);
+        qkv_tile_lds<BM, BN, TM, TN, WVM, QNI>(acc, (float *)lds0, (float *)lds1, m0, n0, wm, wn, e,
+                                               QPRE ? &qpre : nullptr, kg == 0);
         return;
     }
     if (KG > 1 && kg > 0) return;   /* (no barrier below for the store epilogue) */
@@ -806,7 +814,7 @@ __global__ void __launch_bounds__(64 * WVM * WVN * KG) k_gemm_tile(const u16 *__
 #pragma unroll
         for (int j = 0; j < TN; j++)
             epilogue_tile<E>(acc[i][j], m0 + wm * WM + i * 32, n0 + wn * WN + j * 32, e,
-                             XPRE ? xpre : nullptr);
+                             XPRE ? xpre[XPRE ? i * TN + j : 0] : nullptr);
 }
 
 /* ---- per-row RMSNorm ------------------------------------------------------------ */
@@ -1121,7 +1129,7 @@ static void launch_tile(hipStream_t s, const uint16_t *A, int lda, const uint16_
                         int K, const EpiArgs &e)
 {
     const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
-    if constexpr (BM == 256 && E != EPI_QKV) {   /* eight waves (4 x 2): two per SIMD */
+    if constexpr (BM >= 128) {   /* eight waves (4 x 2): two per SIMD */
         hipLaunchKernelGGL((k_gemm_tile<BM, BN, E, 3, 4, RS>), dim3(tm * tn), dim3(512), 0, s, (const u16 *)A,
                            lda, (const u16 *)W, K, K, e, tm, tn);
     } else if constexpr (BM == 32 && BN == 32) {   /* one wave (per K group) */
@@ -1140,6 +1148,9 @@ static void launch_tile(hipStream_t s, const uint16_t *A, int lda, const uint16_
         else
             hipLaunchKernelGGL((k_gemm_tile<BM, BN, E, ring_depth<BM, BN>(true, E == EPI_GATE), 1, RS>), dim3(tm * tn),
                                dim3(128), 0, s, (const u16 *)A, lda, (const u16 *)W, K, K, e, tm, tn);
+    } else if constexpr (BN == 128) {              /* 64 x 128, prefill rows */
+        hipLaunchKernelGGL((k_gemm_tile<BM, BN, E, 3, 2, RS>), dim3(tm * tn), dim3(GT), 0, s, (const u16 *)A,
+                           lda, (const u16 *)W, K, K, e, tm, tn);
     } else {
         if (M <= 64 && BM == 64)
             hipLaunchKernelGGL((k_gemm_tile<BM, BN, E, ring_depth<BM, BN>(true), 2, RS>), dim3(tm * tn),
@@ -1177,11 +1188,53 @@ static void launch_tile_split(hipStream_t s, const uint16_t *A, int lda, const u
                            (const u16 *)A, lda, (const u16 *)W, K, K / ns, e, tm, tn);
 }
 
+/* Tile of a GEMM of more than 64 rows: the one with the least modelled time,
+ *   fixed + stages * max(floor, slope * ceil(tiles / 256 CUs)) microseconds,
+ * stages = K / 64, fitted to every tile on 19 shapes of the Stories and scaled
+ * models (512-2048 rows, N 768-11264, K 768-5632; random data, 10 launches
+ * back to back, best of 5; the fit is within 12% where the choice lies):
+ *   tile               fixed  floor  slope   per CU  waves
+ *   64 x 64 (4 waves)   2.5   0.33   0.235     3      12
+ *   64 x 128 (4)        2.7   0.40   0.36      2       8
+ *   128 x 128 (8)       3.7   0.60   0.60      1       8
+ *   256 x 128 (8)       5.0   1.05   1.05      1       8
+ * Small tiles start and end sooner and quantise finer; large ones move fewer
+ * operand bytes per product through L2 and LDS.  Measured (us) where 64 x 64
+ * was used before, 64 x 64 / 64 x 128 / 128 x 128 / 256 x 128:
+ *   1900 x 2048 x 5632   94.8 / 60.5 / 56.2 / 80.3
+ *   1900 x 2048 x 2048   31.6 / 24.0 / 22.8 / 33.2
+ *   1900 x 4096 x 2048   60.6 / 45.2 / 42.6 / 39.8
+ *   1024 x 2048 x 2048   16.2 / 15.2 / 18.6 / 29.6
+ *   512 x 11264 x 2048   38.3 / 34.5 / 36.8 / 34.5
+ *   2048 x 2304 x 768    16.0 / 17.0 / 18.0 / 16.9
+ *   2048 x 768 x 768      7.3 /  7.5 /  8.9 / 13.9
+ * A 1900-token prompt through four layers of the 2048-wide GQA model: 1605 ->
+ * 1289 us, the same logits bit for bit.  The QKV epilogue is not built for
+ * 64 x 128. */
+enum { TILE_64x64, TILE_64x128, TILE_128x128, TILE_256x128 };
+
+static int pick_tile(int M, int N, int K, bool qkv)
+{
+    static const struct { int bm, bn; float fixed, floor, slope; } T[4] = {
+        {64, 64, 2.5f, 0.33f, 0.235f},
+        {64, 128, 2.7f, 0.40f, 0.36f},
+        {128, 128, 3.7f, 0.60f, 0.60f},
+        {256, 128, 5.0f, 1.05f, 1.05f}};
+    int best = TILE_64x64;
+    float tb = 0.f;
+    for (int i = TILE_64x64; i <= TILE_256x128; i++) {
+        if (i == TILE_64x128 && qkv) continue;
+        const long tiles = (long)((M + T[i].bm - 1) / T[i].bm) * ((N + T[i].bn - 1) / T[i].bn);
+        const float per = T[i].slope * (float)((tiles + 255) / 256);
+        const float t = T[i].fixed + (float)(K / BKH) * (per > T[i].floor ? per : T[i].floor);
+        if (i == TILE_64x64 || t < tb) { best = i; tb = t; }
+    }
+    return best;
+}
+
 /* Tile choice (measured on MI355X over the Stories and scaled-model shapes):
- * 64 x 64 tiles everywhere, since four of them share a CU and hide each
- * other's latency, except for GEMMs big enough to give every CU a 256 x 128
- * tile (classifiers, the 2048-row W1/W3), where the larger tile's lower L2
- * traffic wins; a decode-row classifier (N >= 16384, which cannot be K-split
+ * more than 64 rows follow pick_tile.  Up to 64 rows take 64 x 64 tiles,
+ * except: a decode-row classifier (N >= 16384, which cannot be K-split
  * ahead of its argmax) takes 64 x 64 tiles, twice the work-groups of 64 x 128
  * (C2 0.4480 -> 0.4434, C4 1.148 -> 1.142 ms/step; 32 x 64 lost at C2);
  * up to 32 rows take 32 x 64 tiles of two waves (a 64-row tile would stage and
@@ -1211,24 +1264,28 @@ static int launch_gemm(hipStream_t s, const uint16_t *A, int lda, const uint16_t
                        int K, const EpiArgs &e)
 {
     if (K % BKH) return hipErrorInvalidValue;
-    if constexpr (RS) {
-        /* row-scaled GEMMs (prefill rows): the two prefill tiles, but QKV only
-         * on 64 x 64 (its four-wave 256 x 128 tile with the row scale used
-         * in-flight LDS read registers early; the assembly check rejects it) */
-        if (E == EPI_GATE && (long)((M + 255) / 256) * ((N + 127) / 128) >= 240) {
-            if constexpr (E == EPI_GATE) launch_tile<256, 128, E, true>(s, A, lda, W, M, N, K, e);
-        } else launch_tile<64, 64, E, true>(s, A, lda, W, M, N, K, e);
-    } else if (M <= 64 && N >= 16384) {
-        /* decode-row classifiers (and any other wide decode-row GEMM, the
-         * QKV epilogue included) on 64 x 64 tiles */
-        launch_tile<64, 64, E>(s, A, lda, W, M, N, K, e);
+    if (M <= 64) {
+        if constexpr (RS) {
+            launch_tile<64, 64, E, true>(s, A, lda, W, M, N, K, e);
+        } else if (N >= 16384) {
+            /* decode-row classifiers (and any other wide decode-row GEMM, the
+             * QKV epilogue included) on 64 x 64 tiles */
+            launch_tile<64, 64, E>(s, A, lda, W, M, N, K, e);
+        } else if (E == EPI_GATE && (long)((M + 31) / 32) * ((N + 63) / 64) <= 128) {
+            if constexpr (E == EPI_GATE) launch_tile<32, 32, E>(s, A, lda, W, M, N, K, e);
+        } else if (E != EPI_QKV && (M <= 32 || E == EPI_GATE)) {
+            if constexpr (E != EPI_QKV) launch_tile<32, 64, E>(s, A, lda, W, M, N, K, e);
+        } else launch_tile<64, 64, E>(s, A, lda, W, M, N, K, e);
+        return hipGetLastError();
     }
-    else if ((long)((M + 255) / 256) * ((N + 127) / 128) >= 240) launch_tile<256, 128, E>(s, A, lda, W, M, N, K, e);
-    else if (E == EPI_GATE && M <= 64 && (long)((M + 31) / 32) * ((N + 63) / 64) <= 128) {
-        if constexpr (E == EPI_GATE) launch_tile<32, 32, E>(s, A, lda, W, M, N, K, e);
-    } else if (E != EPI_QKV && (M <= 32 || (E == EPI_GATE && M <= 64))) {
-        if constexpr (E != EPI_QKV) launch_tile<32, 64, E>(s, A, lda, W, M, N, K, e);
-    } else launch_tile<64, 64, E>(s, A, lda, W, M, N, K, e);
+    switch (pick_tile(M, N, K, E == EPI_QKV)) {
+    case TILE_256x128: launch_tile<256, 128, E, RS>(s, A, lda, W, M, N, K, e); break;
+    case TILE_128x128: launch_tile<128, 128, E, RS>(s, A, lda, W, M, N, K, e); break;
+    case TILE_64x128:
+        if constexpr (E != EPI_QKV) launch_tile<64, 128, E, RS>(s, A, lda, W, M, N, K, e);
+        break;
+    default: launch_tile<64, 64, E, RS>(s, A, lda, W, M, N, K, e);
+    }
     return hipGetLastError();
 }
 
