@@ -483,12 +483,28 @@ struct QkvPart {
     KT *kc, *vc;            /* the cache, written at the current position */
 };
 
-template <int HD, typename KT>
+/* A head's positions split over ns work-groups (SPL): work-group sp takes the
+ * tiles of waves sp*4 .. sp*4+3 of 4*ns; all but the last hand their running
+ * (sum, max, weighted V) to it as tagged words w[sp][HD + 2] (the sums of V,
+ * then max, then sum), and the last one merges them and the current position.
+ * The last is also last in dispatch order, so that it waits only for
+ * work-groups before it. */
+struct SplitPart {
+    unsigned long long *w;
+    int sp, ns;
+};
+
+template <int HD, typename KT, bool SPL = false>
 __device__ __forceinline__ void attn_head(
     const float *__restrict__ q, const KT *__restrict__ kc, const KT *__restrict__ vc,
     const int *__restrict__ pos, const int *__restrict__ slot, int H, int Hkv, int max_seq,
-    float *oh, int h, int b, const QkvPart<KT> *qp = nullptr, const QkvTagged *qt = nullptr)
+    float *oh, int h, int b, const QkvPart<KT> *qp = nullptr, const QkvTagged *qt = nullptr,
+    const SplitPart *sq = nullptr)
 {
+    /* this wave's place among the TS waves that take the tiles in turn, and
+     * whether this work-group writes the head output */
+    const bool fin = !SPL || sq->sp == sq->ns - 1;
+    const int TS = SPL ? NWAVE * sq->ns : NWAVE;
     /* positions per tile: 32 (measured against 64: the four waves share short
      * contexts more evenly).  Two tiles fit the registers except at hd 128 with
      * an fp32 cache, so the next tile's K/V loads are in flight while the
@@ -503,7 +519,8 @@ __device__ __forceinline__ void attn_head(
     __shared__ __attribute__((aligned(16))) float so[NWAVE][HD];
     __shared__ __attribute__((aligned(16))) float sqkv[3][HD];   /* q, k, v of a split QKV */
     __shared__ float scur;                                        /* its current score */
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wl = threadIdx.x >> 6;
+    const int wv = SPL ? wl + NWAVE * sq->sp : wl;                  /* first tile */
     const int ctx = pos[b] + 1;
     /* positions read from the cache: all of them, or with qp / qt all but the
      * current one, which is added from LDS at the end */
@@ -576,7 +593,7 @@ __device__ __forceinline__ void attn_head(
             if (qt) {
 #pragma unroll
                 for (int i = 0; i < NP; i++) {
-                    const int p = min((wv + NWAVE) * TILE + pp + PP * i, max_seq - 1);
+                    const int p = min((wv + TS) * TILE + pp + PP * i, max_seq - 1);
                     kv_raw_load(K + (size_t)p * HD, kr1[i]);
                     kv_raw_load(V + (size_t)p * HD, vr1[i]);
                 }
@@ -676,6 +693,7 @@ __device__ __forceinline__ void attn_head(
          * that gives up sets qt->err, and the kernel still ends) */
         const unsigned tag = qkv_tag(*qt);
         const int g = small_div(h, small_div(H, Hkv));
+        const int nw = fin ? 3 * HD : HD;    /* only the last split needs k and v */
         constexpr int NT = (3 * HD + WG - 1) / WG;
         const unsigned long long *wp[NT];
         unsigned long long v[NT];
@@ -684,12 +702,12 @@ __device__ __forceinline__ void attn_head(
             const int t = threadIdx.x + j * WG, vec = t / HD, e = t % HD;
             wp[j] = vec == 0 ? qt->tq + (size_t)b * H * HD + h * HD + e
                              : (vec == 1 ? qt->tk : qt->tv) + (size_t)b * Hkv * HD + g * HD + e;
-            v[j] = t < 3 * HD ? tag_peek(wp[j]) : 0ull;
+            v[j] = t < nw ? tag_peek(wp[j]) : 0ull;
         }
 #pragma unroll
         for (int j = 0; j < NT; j++) {
             const int t = threadIdx.x + j * WG;
-            if (t < 3 * HD) sqkv[t / HD][t % HD] = tag_take(v[j], wp[j], tag, qt->err);
+            if (t < nw) sqkv[t / HD][t % HD] = tag_take(v[j], wp[j], tag, qt->err);
         }
     }
     if (cur) {
@@ -699,7 +717,7 @@ __device__ __forceinline__ void attn_head(
         /* the current position's score, its k rounded as the cache would, by
          * the last wave (tiles go to the waves in turn, so it has the fewest);
          * it is read only at the merge, after the barrier */
-        if (wv == NWAVE - 1) {
+        if (wl == NWAVE - 1 && fin) {
             float d = 0.f;
 #pragma unroll
             for (int j = lane; j < HD; j += 64) d = fmaf(sqkv[0][j], kv_round<KT>(sqkv[1][j]), d);
@@ -780,8 +798,8 @@ __device__ __forceinline__ void attn_head(
              * time (contexts past 8 tiles) */
             if (wv < ntiles) {                                   /* wave-uniform */
                 consume(wv, ck[0], cv[0]);
-                if (wv + NWAVE < ntiles) consume(wv + NWAVE, ck[PRECVT ? 1 : 0], cv[PRECVT ? 1 : 0]);
-                for (int t = wv + 2 * NWAVE; t < ntiles; t += NWAVE) {
+                if (wv + TS < ntiles) consume(wv + TS, ck[PRECVT ? 1 : 0], cv[PRECVT ? 1 : 0]);
+                for (int t = wv + 2 * TS; t < ntiles; t += TS) {
                     fetch(t, kr, vr);
                     consume(t, kr, vr);
                 }
@@ -792,22 +810,22 @@ __device__ __forceinline__ void attn_head(
              * the loop's registers at two tiles (143 -> 109 VGPRs at hd 64).
              * The scheduling barriers keep each fetch ahead of the compute it
              * overlaps (the compiler would sink the loads to their first use). */
-            if (!qt) fetch(wv + NWAVE, kr1, vr1);
+            if (!qt) fetch(wv + TS, kr1, vr1);
             __builtin_amdgcn_sched_barrier(0);
             if (wv < ntiles) {                                   /* wave-uniform */
                 consume(wv, kr, vr);
-                for (int t = wv + NWAVE; t < ntiles; t += 2 * NWAVE) {   /* kr1: tile t */
-                    fetch(t + NWAVE, kr, vr);
+                for (int t = wv + TS; t < ntiles; t += 2 * TS) {   /* kr1: tile t */
+                    fetch(t + TS, kr, vr);
                     __builtin_amdgcn_sched_barrier(0);
                     consume(t, kr1, vr1);
-                    if (t + NWAVE >= ntiles) break;
-                    fetch(t + 2 * NWAVE, kr1, vr1);
+                    if (t + TS >= ntiles) break;
+                    fetch(t + 2 * TS, kr1, vr1);
                     __builtin_amdgcn_sched_barrier(0);
-                    consume(t + NWAVE, kr, vr);
+                    consume(t + TS, kr, vr);
                 }
             }
         } else {
-            for (int t = wv; t < ntiles; t += NWAVE) {      /* wave-uniform */
+            for (int t = wv; t < ntiles; t += TS) {      /* wave-uniform */
                 if (t != wv) fetch(t, kr, vr);
                 consume(t, kr, vr);
             }
@@ -818,21 +836,45 @@ __device__ __forceinline__ void attn_head(
     for (int j = 0; j < 8; j++) o[j] = across(o[j], fadd);
     if (lane < G) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) so[wv][dq * 8 + j] = o[j];
+        for (int j = 0; j < 8; j++) so[wl][dq * 8 + j] = o[j];
     }
-    if (lane == 0) { sm[wv] = m; sl[wv] = l; }
+    if (lane == 0) { sm[wl] = m; sl[wl] = l; }
+    /* the other splits' (V sums, max, sum), fetched before the barrier */
+    __shared__ float sps[SPL ? (LM_ATTN_SPLIT_MAX - 1) * (HD + 2) : 1];
+    if constexpr (SPL) {
+        if (fin) tag_wait_span(sq->w, (sq->ns - 1) * (HD + 2), qkv_tag(*qt), qt->err, sps);
+    }
     __syncthreads();
     if (threadIdx.x < HD) {
         const int d = threadIdx.x;
-        float M = cur ? scur : -INFINITY;
+        float M = cur && fin ? scur : -INFINITY;
 #pragma unroll
         for (int w = 0; w < NWAVE; w++) M = fmaxf(M, sm[w]);
+        if constexpr (SPL) {
+            if (fin)
+                for (int s = 0; s < sq->ns - 1; s++) M = fmaxf(M, sps[s * (HD + 2) + HD]);
+        }
         float L = 0.f, acc = 0.f;
 #pragma unroll
         for (int w = 0; w < NWAVE; w++) {
             const float f = sm[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sm[w] - M);
             L = fmaf(sl[w], f, L);
             acc = fmaf(so[w][d], f, acc);
+        }
+        if constexpr (SPL) {
+            if (!fin) {   /* this split's share, for the last one to merge */
+                const unsigned tag = qkv_tag(*qt);
+                unsigned long long *w = sq->w + (size_t)sq->sp * (HD + 2);
+                tag_store(w + d, acc, tag);
+                if (d < 2) tag_store(w + HD + d, d == 0 ? M : L, tag);
+                return;
+            }
+            for (int s = 0; s < sq->ns - 1; s++) {
+                const float *ps = sps + s * (HD + 2);
+                const float f = ps[HD] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ps[HD] - M);
+                L = fmaf(ps[HD + 1], f, L);
+                acc = fmaf(ps[d], f, acc);
+            }
         }
         if (cur) {   /* the current position, after the cached ones */
             const float f = __builtin_amdgcn_exp2f(scur - M);
@@ -841,6 +883,7 @@ __device__ __forceinline__ void attn_head(
         }
         oh[d] = acc / L;
     }
+    if (SPL && !fin) return;
     __syncthreads();
 }
 
@@ -1060,11 +1103,19 @@ struct FfnArgs {
     const u16 *w2;        /* [D, F] */
 };
 
+/* Split attention (SPL): work-groups per head, and their hand-off words. */
+template <bool SPL> struct SplitArgs {};
+template <> struct SplitArgs<true> {
+    unsigned long long *w;   /* [row * H + head][LM_ATTN_SPLIT_MAX - 1][hd + 2] */
+    int ns;
+};
+
 /* One launch of the batch 1-4 decode chain per layer; its work-groups take
  * roles in this order, each role waiting only on roles before it:
  *  - 0 .. nprod-1: the QKV GEMV of k_qkv_rope, also storing q, k, v as tagged
  *    hand-off words;
- *  - then one per (row b, head h): the attention of head h, row b, which loads
+ *  - then one (SPL: ns, the positions split over them) per (row b, head h): the
+ *    attention of head h, row b, which loads
  *    its first cached K/V tile, waits for the current position's q, k, v words
  *    and hands the head output on (fp32 to out[b, h*HD ..] without WO, else
  *    as tagged words, in LM_TA_COPIES copies);
@@ -1079,15 +1130,16 @@ struct FfnArgs {
  * launch; the QKV and Wo work-groups read x before they store any word, and x
  * is written only after every word of every head, so no read of x in the
  * launch sees the value written in it. */
-template <int D, int NB, typename KT, int HD, bool WO, int F>
+template <int D, int NB, typename KT, int HD, bool WO, int F, bool SPL>
 __global__ void __launch_bounds__(WG) k_qkv_attn(
     float *__restrict__ x, const u16 *__restrict__ emb, const int *__restrict__ tok,
     const float *__restrict__ rms_w, const u16 *__restrict__ W, int NQ, int NKV,
     const float *__restrict__ rc, const float *__restrict__ rs, const int *__restrict__ pos,
     int B, KT *__restrict__ kc, KT *__restrict__ vc, int max_seq, int npairs, int nprod, int H,
-    QkvTagged tg, float *__restrict__ out, const u16 *__restrict__ Wo, FfnArgs ffn)
+    QkvTagged tg, float *__restrict__ out, const u16 *__restrict__ Wo, FfnArgs ffn, SplitArgs<SPL> sa)
 {
     static_assert(F == 0 || WO, "the FFN roles take x' from the Wo role");
+    static_assert(!SPL || WO, "split heads hand on to the Wo role");
     static_assert(LM_TA_COPIES <= 64 && LM_TX_COPIES <= 64 && LM_TG_COPIES <= 64, "a wave's lanes store the copies");
     if ((int)blockIdx.x < nprod) {
         qkv_rows<D, NB, KT>(x, emb, tok, rms_w, W, NQ, NKV, HD, rc, rs, pos, B, nullptr, kc, vc,
@@ -1095,10 +1147,22 @@ __global__ void __launch_bounds__(WG) k_qkv_attn(
         return;
     }
     int a = blockIdx.x - nprod;
-    if (!WO || a < H * B) {
+    int nattn = H * B;
+    if constexpr (SPL) nattn *= sa.ns;
+    if (!WO || a < nattn) {
         __shared__ float oh[HD];
-        const int h = a % H, b = a / H;
-        attn_head<HD, KT>(nullptr, kc, vc, pos, nullptr, H, NKV / HD, max_seq, oh, h, b, nullptr, &tg);
+        int r = a;
+        if constexpr (SPL) r = a % (H * B);
+        const int h = r % H, b = r / H;
+        if constexpr (SPL) {
+            /* split a / (H*B): the heads' last splits come last */
+            const SplitPart sq = {sa.w + (size_t)r * ((LM_ATTN_SPLIT_MAX - 1) * (HD + 2)), a / (H * B), sa.ns};
+            attn_head<HD, KT, true>(nullptr, kc, vc, pos, nullptr, H, NKV / HD, max_seq, oh, h, b,
+                                           nullptr, &tg, &sq);
+            if (sq.sp != sq.ns - 1) return;
+        } else {
+            attn_head<HD, KT>(nullptr, kc, vc, pos, nullptr, H, NKV / HD, max_seq, oh, h, b, nullptr, &tg);
+        }
         if constexpr (WO) {
             /* every copy of the head output, the work-group's threads taking
              * (element, copy) pairs */
@@ -1118,7 +1182,7 @@ __global__ void __launch_bounds__(WG) k_qkv_attn(
         constexpr int ROW = F > D ? F : D;
         __shared__ __attribute__((aligned(16))) float xs[NB * ROW];
         constexpr int NWO = (D / 2 + NWAVE - 1) / NWAVE;
-        a -= H * B;
+        a -= nattn;
         if (F == 0 || a < NWO) {
             wo_role<D, NB, F>(x, emb, tok, Wo, B, NQ, tg, a, xs);
             return;
@@ -1561,46 +1625,59 @@ extern "C" int lmk_qkv_attn(hipStream_t s, float *x, const uint16_t *emb, const 
                             unsigned long long *tagged, const unsigned *epoch, int layer,
                             int n_layers, int *err, float *out, const uint16_t *wo,
                             const float *rms_ffn, const uint16_t *w13, const uint16_t *w2, int F,
-                            int wgs_per_cu)
+                            int wgs_per_cu, int nsplit)
 {
     if (B < 1 || B > 4 || NQ != D || H < 1 || NQ != H * hd || NKV % hd || H % (NKV / hd) ||
         (emb && !tok) || !tagged || !epoch || !err || (!out && !wo) || (hd != 64 && hd != 128) ||
+        nsplit < 1 || nsplit > LM_ATTN_SPLIT_MAX ||
         (w13 && (!wo || !w2 || !rms_ffn || F < 1 || F % LMK_GATE_BLOCK || !lmk_layer_fusable(D, F, B))))
         return hipErrorInvalidValue;
     const int npairs = (NQ + 2 * NKV) / 2;
     const int nprod = (npairs + NWAVE - 1) / NWAVE;
     const int nwo = wo ? (D / 2 + NWAVE - 1) / NWAVE : 0;
-    dim3 grid(nprod + H * B + nwo);   /* with the FFN: + its roles' work-groups, below */
+    /* split heads: with the Wo role, and in the whole-layer form at one row
+     * (the batches it runs by default) */
+    const bool split = nsplit > 1 && wo && (!w13 || B == 1);
+    dim3 grid(nprod + H * B * (split ? nsplit : 1) + nwo);   /* with the FFN: + its roles' work-groups, below */
     unsigned long long *ta = tagged + (size_t)LM_TAG_B * (NQ + 2 * NKV);
     unsigned long long *tx = ta + (size_t)LM_TA_COPIES * LM_TAG_B * NQ;
     unsigned long long *tgt = tx + (size_t)LM_TX_COPIES * LM_TAG_B * D;
+    unsigned long long *tsp = tgt + (size_t)LM_TG_COPIES * LM_TAG_B * F;
     const QkvTagged tg = {tagged, tagged + (size_t)LM_TAG_B * NQ, tagged + (size_t)LM_TAG_B * (NQ + NKV),
                           ta, tx, tgt, epoch, layer, n_layers, err};
     const FfnArgs ffn = {rms_ffn, (const u16 *)w13, (const u16 *)w2};
-#define LAUNCH_QA(HD_, KT_, WO_, F_)                                                                 \
+    SplitArgs<true> sa_true = {tsp, nsplit};
+    SplitArgs<false> sa_false;
+#define LAUNCH_QA(HD_, KT_, WO_, F_, SPL_)                                                           \
     do {                                                                                             \
-        const size_t shm_ = F_ ? lds_cap_pad<k_qkv_attn<K_, NB_, KT_, HD_, WO_, F_>>(wgs_per_cu) : 0; \
-        DLAUNCH((k_qkv_attn<K_, NB_, KT_, HD_, WO_, F_>), grid, dim3(WG), shm_, s, x, emb, tok, rms_w, \
+        const size_t shm_ = F_ ? lds_cap_pad<k_qkv_attn<K_, NB_, KT_, HD_, WO_, F_, SPL_>>(wgs_per_cu) : 0; \
+        DLAUNCH((k_qkv_attn<K_, NB_, KT_, HD_, WO_, F_, SPL_>), grid, dim3(WG), shm_, s, x, emb, tok, rms_w, \
                 wqkv, NQ, NKV, rope_cos, rope_sin, pos, B, (KT_ *)kc, (KT_ *)vc, max_seq, npairs,      \
-                nprod, H, tg, out, (const u16 *)wo, ffn);                                            \
+                nprod, H, tg, out, (const u16 *)wo, ffn, sa_##SPL_);                                 \
     } while (0)
-#define LAUNCH_QA_KV(WO_, F_)                                    \
-    do {                                                         \
-        if (hd == 64 && kv_f32) LAUNCH_QA(64, float, WO_, F_);   \
-        else if (hd == 64) LAUNCH_QA(64, u16, WO_, F_);          \
-        else if (kv_f32) LAUNCH_QA(128, float, WO_, F_);         \
-        else LAUNCH_QA(128, u16, WO_, F_);                       \
+#define LAUNCH_QA_KV(WO_, F_, SPL_)                                    \
+    do {                                                               \
+        if (hd == 64 && kv_f32) LAUNCH_QA(64, float, WO_, F_, SPL_);   \
+        else if (hd == 64) LAUNCH_QA(64, u16, WO_, F_, SPL_);          \
+        else if (kv_f32) LAUNCH_QA(128, float, WO_, F_, SPL_);         \
+        else LAUNCH_QA(128, u16, WO_, F_, SPL_);                       \
     } while (0)
     if (w13) {
         DISPATCH_DF(D, F, DISPATCH_NB(B, {
             grid.x += (F_ + NWAVE - 1) / NWAVE + (K_ / 2 + NWAVE - 1) / NWAVE;
-            LAUNCH_QA_KV(true, F_);
+            if constexpr (NB_ == 1) {
+                if (split) LAUNCH_QA_KV(true, F_, true);
+                else LAUNCH_QA_KV(true, F_, false);
+            } else {
+                LAUNCH_QA_KV(true, F_, false);
+            }
         }));
     } else {
         DISPATCH_D(D, DISPATCH_NB(B, {
             if (!GEMV_LDS_OK(K_, NB_)) return hipErrorInvalidValue;
-            if (wo) LAUNCH_QA_KV(true, 0);
-            else LAUNCH_QA_KV(false, 0);
+            if (split) LAUNCH_QA_KV(true, 0, true);
+            else if (wo) LAUNCH_QA_KV(true, 0, false);
+            else LAUNCH_QA_KV(false, 0, false);
         }));
     }
 #undef LAUNCH_QA_KV

@@ -88,8 +88,13 @@ int lmk_qkv_rope(hipStream_t s, float *x, const uint16_t *emb, const int *tok,
 #ifndef LM_TG_COPIES
 #define LM_TG_COPIES 1
 #endif
+/* Most work-groups that one head's positions are split over in the batch 1-4
+ * chain; the words of the split partials follow the others: (hd + 2) per
+ * split but the last, row and head (hd >= 64, so at most NQ/32 beside NQ). */
+#define LM_ATTN_SPLIT_MAX 16
 #define LM_TAG_WORDS(NQ, NKV, D, F) \
-    ((size_t)LM_TAG_B * ((NQ) + 2 * (NKV) + LM_TA_COPIES * (NQ) + LM_TG_COPIES * (F) + LM_TX_COPIES * (D)))
+    ((size_t)LM_TAG_B * ((NQ) + 2 * (NKV) + LM_TA_COPIES * (NQ) + LM_TG_COPIES * (F) + LM_TX_COPIES * (D) + \
+                         (LM_ATTN_SPLIT_MAX - 1) * ((NQ) + (NQ) / 32)))
 
 /* lmk_qkv_rope and the attention of every (head, row) in one launch: the
  * QKV work-groups hand q, k, v of the current position to the attention
@@ -107,7 +112,8 @@ int lmk_qkv_rope(hipStream_t s, float *x, const uint16_t *emb, const int *tok,
  * 128.  wgs_per_cu (1-4; 0 = as registers and LDS allow): at most that many
  * work-groups of the whole-layer launch share a CU, enforced with dynamic
  * LDS, so the later roles' work-groups (W1/W3, W2) are dispatched as the
- * early ones finish instead of all at once. */
+ * early ones finish instead of all at once.  nsplit (1 .. LM_ATTN_SPLIT_MAX):
+ * work-groups that share a head's positions (with wo; with w13 at one row). */
 int lmk_qkv_attn(hipStream_t s, float *x, const uint16_t *emb, const int *tok,
                  const float *rms_w, const uint16_t *wqkv, int D, int NQ, int NKV, int hd,
                  const float *rope_cos, const float *rope_sin, const int *pos, int B,
@@ -115,7 +121,7 @@ int lmk_qkv_attn(hipStream_t s, float *x, const uint16_t *emb, const int *tok,
                  unsigned long long *tagged, const unsigned *epoch, int layer,
                  int n_layers, int *err, float *out, const uint16_t *wo,
                  const float *rms_ffn, const uint16_t *w13, const uint16_t *w2, int F,
-                 int wgs_per_cu);
+                 int wgs_per_cu, int nsplit);
 
 /* Whether the whole-layer form of lmk_qkv_attn (w13 given) is built for this
  * model width, hidden width and batch. */

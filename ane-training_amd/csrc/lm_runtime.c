@@ -36,6 +36,7 @@
 
 #define MAX_GEMV_B 4
 #define PREFILL_GRAPHS 4   /* prefill chunk shapes kept captured */
+#define CTX_CLASSES 4      /* context lengths the decode attention is launched for (ctx_class) */
 
 struct LMModel {
     Config cfg;                 /* vocab_size positive */
@@ -87,7 +88,7 @@ struct LMModel {
     int *h_io;
     /* captured decode graphs: [B][0] one step, [B][1] GRAPH_STEPS steps
      * (greedy feedback stays on the device) */
-    hipGraphExec_t (*step_graph)[2];   /* [max_batch + 1][2]   */
+    hipGraphExec_t (*step_graph)[2][CTX_CLASSES];   /* [max_batch + 1][2][context class] */
     /* captured prefill chunks (the layers and, with all logits, the
      * classifier), by rows, rows per sequence and logits mode; replaced round
      * robin */
@@ -97,6 +98,7 @@ struct LMModel {
     } pgraph[PREFILL_GRAPHS];
     int pgraph_next;
     int use_graph;
+    int ctx_cls;                /* context class of the decode step being queued */
 };
 
 static int g_init_status = 1; /* 1 = not attempted */
@@ -328,11 +330,13 @@ static void drop_graphs(LMModel *m)
         }
     if (!m->step_graph) return;
     for (int b = 0; b <= m->max_batch; b++)
-        for (int k = 0; k < 2; k++)
-            if (m->step_graph[b][k]) {
-                hipGraphExecDestroy(m->step_graph[b][k]);
-                m->step_graph[b][k] = NULL;
+        for (int k = 0; k < 2 * CTX_CLASSES; k++) {
+            hipGraphExec_t *ge = &m->step_graph[b][k / CTX_CLASSES][k % CTX_CLASSES];
+            if (*ge) {
+                hipGraphExecDestroy(*ge);
+                *ge = NULL;
             }
+        }
 }
 
 static void free_rows(LMModel *m)
@@ -492,7 +496,7 @@ static LMModel *create_model(const Config *cfg, const WSrc *w, int max_batch, in
     m->layer_elems = m->off_w2 + D * F;
     m->kv_layer_elems = (size_t)max_batch * m->Hkv * max_seq * m->hd;
     const size_t NB = (size_t)max_batch;
-    m->step_graph = (hipGraphExec_t(*)[2])calloc(NB + 1, sizeof(*m->step_graph));
+    m->step_graph = (hipGraphExec_t(*)[2][CTX_CLASSES])calloc(NB + 1, sizeof(*m->step_graph));
     if (!m->step_graph) FAIL(LM_ERR_OOM);
 
     if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) FAIL(LM_ERR_HIP);
@@ -770,6 +774,34 @@ static int chain_level(const LMModel *m, int B)
     return lvl == 3 && !lmk_layer_fusable(m->D, m->F, B) ? 2 : lvl;
 }
 
+/* Context class of batch 1-4 decode rows whose largest position is p: class 0
+ * up to 512 cached positions, then one more per doubling (the last for any
+ * more).  From class 1 the chain splits a head's positions over attn_split
+ * work-groups, so that each of their waves has at most two tiles of 32, which
+ * it holds before its wait for q, k, v.  One work-group per head stays up to
+ * 512: with two, the whole-layer launch of Stories measured 12.6 against 12.1
+ * us at 350 positions and 12.6 against 12.8 at 500 (the merge costs one more
+ * hand-off), while 1900 positions took 23.6 us unsplit and 14.3 split over 8.
+ * The class is fixed when a graph is captured, so each has its own graph. */
+static int ctx_class(int p)
+{
+    int c = 0;
+    while (c < CTX_CLASSES - 1 && p > (512 << c)) c++;
+    return c;
+}
+
+static int ctx_class_rows(const int *pos, int B, int more)
+{
+    int p = 0;
+    if (B > MAX_GEMV_B) return 0;   /* (the MFMA path has one form) */
+    for (int b = 0; b < B; b++)
+        if (pos[b] > p) p = pos[b];
+    return ctx_class(p + more);
+}
+
+/* Work-groups per head of a context class: 1, 4, 8, 16. */
+static int attn_split(int cls) { return cls ? 2 << cls : 1; }
+
 /* Whether kernel family fam runs inside another family's launch at fusion
  * level lvl (the QKV launch; at level 3 the argmax inside the classifier's). */
 static int fam_inside(int fam, int lvl)
@@ -798,7 +830,7 @@ static int enqueue_kernel(LMModel *m, int B, int fam, int l, float *logits)
                               m->max_seq, m->H, m->d_tagged, m->d_epoch, l, m->L, m->d_err,
                               m->d_attn, lvl >= 2 ? lw + m->off_wo : NULL,
                               m->d_rms_ffn + (size_t)l * D, lvl == 3 ? lw + m->off_w13 : NULL,
-                              lw + m->off_w2, F, m->layer_wgs));
+                              lw + m->off_w2, F, m->layer_wgs, attn_split(m->ctx_cls)));
         else
             KCHK(lmk_qkv_rope(s, m->d_x, l == 0 ? m->d_embed : NULL, m->d_tok,
                               m->d_rms_att + (size_t)l * D, lw, D, m->NQ, m->NKV, m->hd,
@@ -1036,7 +1068,7 @@ static int enqueue_decode_steps(LMModel *m, int B, int nsteps)
         }
         return LM_OK;
     }
-    hipGraphExec_t *ge = &m->step_graph[B][nsteps == 1 ? 0 : 1];
+    hipGraphExec_t *ge = &m->step_graph[B][nsteps == 1 ? 0 : 1][m->ctx_cls];
     if (!*ge) {
         hipGraph_t g;
         HIPCHK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
@@ -1061,8 +1093,9 @@ static int step_waits(const LMModel *m, int B)
     return B <= MAX_GEMV_B && chain_level(m, B) >= 1;
 }
 
-static int run_decode_steps(LMModel *m, int B, int nsteps)
+static int run_decode_steps(LMModel *m, int B, int nsteps, int cls)
 {
+    m->ctx_cls = cls;
     if (B > MAX_GEMM_B) {
         fprintf(stderr, "stories_lm: decode batch %d > %d not supported\n", B, MAX_GEMM_B);
         return LM_ERR_UNSUPPORTED;
@@ -1074,7 +1107,6 @@ static int run_decode_steps(LMModel *m, int B, int nsteps)
     return handoff_leave(m, enqueue_decode_steps(m, B, nsteps));
 }
 
-static int run_decode_step(LMModel *m, int B) { return run_decode_steps(m, B, 1); }
 
 /* The hand-off flag of the fused QKV + attention launches: queued to the host
  * with the results of a call, checked once the stream has synchronised. */
@@ -1130,7 +1162,7 @@ int lm_forward_batch(LMModel *m, const int *tokens, const int *pos, int B, float
     memcpy(hio + B, pos, B * 4);
     HIPCHK(hipMemcpyAsync(m->d_tok, hio, B * 4, hipMemcpyHostToDevice, m->stream));
     HIPCHK(hipMemcpyAsync(m->d_pos, hio + B, B * 4, hipMemcpyHostToDevice, m->stream));
-    if ((rc = run_decode_step(m, B))) return rc;
+    if ((rc = run_decode_steps(m, B, 1, ctx_class_rows(pos, B, 0)))) return rc;
     if (argmax)
         HIPCHK(hipMemcpyAsync(hio + 2 * B, m->d_tok, B * 4, hipMemcpyDeviceToHost, m->stream));
     if (logits)
@@ -1157,7 +1189,7 @@ const float *lm_forward(LMModel *m, int token, int pos)
     if (hipMemcpyAsync(m->d_tok, hio, 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
         hipMemcpyAsync(m->d_pos, hio + 1, 4, hipMemcpyHostToDevice, m->stream) != hipSuccess)
         return NULL;
-    if (run_decode_step(m, 1)) return NULL;
+    if (run_decode_steps(m, 1, 1, ctx_class(pos))) return NULL;
     if (hipMemcpyAsync(m->h_logits, m->d_logits, (size_t)m->V * 4, hipMemcpyDeviceToHost,
                        m->stream) != hipSuccess ||
         queue_err_read(m) != LM_OK || hipStreamSynchronize(m->stream) != hipSuccess) {
@@ -1189,9 +1221,9 @@ int lm_generate_greedy(LMModel *m, int B, const int *first_tokens, const int *po
     HIPCHK(hipMemcpyAsync(m->d_pos, hio + B, B * 4, hipMemcpyHostToDevice, m->stream));
     int t = 0;
     for (; t + GRAPH_STEPS <= n_steps; t += GRAPH_STEPS)
-        if ((rc = run_decode_steps(m, B, GRAPH_STEPS))) return rc;
+        if ((rc = run_decode_steps(m, B, GRAPH_STEPS, ctx_class_rows(pos0, B, t + GRAPH_STEPS - 1)))) return rc;
     for (; t < n_steps; t++)
-        if ((rc = run_decode_step(m, B))) return rc;
+        if ((rc = run_decode_steps(m, B, 1, ctx_class_rows(pos0, B, t)))) return rc;
     const size_t stride = (size_t)m->max_seq + 1;
     int *h = (int *)malloc((size_t)B * stride * 4);
     if (!h) return LM_ERR_OOM;
@@ -1481,6 +1513,7 @@ int lm_profile_chain(LMModel *m, int B, const int *tokens, const int *pos, int s
     for (int b = 0; b < B; b++)
         if (pos[b] + steps + 1 > m->max_seq) return LM_ERR_RANGE;
     const int lvl = chain_level(m, B), waits = step_waits(m, B);
+    m->ctx_cls = ctx_class_rows(pos, B, steps);
     /* the launches of one step, in order: (family, layer) */
     const int nmax = 5 * m->L + 2;
     int *kf = (int *)calloc((size_t)nmax, sizeof(int)), *kl = (int *)calloc((size_t)nmax, sizeof(int));
