@@ -459,6 +459,31 @@ __global__ void __launch_bounds__(AT) k_attn_prefill_split(
     }
 }
 
+/* ---- the sequences' last rows ------------------------------------------------ */
+
+/* Work-group i copies sequence i's last residual row and query row: all that
+ * the last layer's attention, Wo and FFN owe a caller that wants the last
+ * rows' logits.  Latency bound (one round trip, n * (D + NQ) * 4 bytes). */
+__global__ void __launch_bounds__(AT) k_last_rows(const float *__restrict__ x, const float *__restrict__ q,
+                                                 int D, int NQ, int S, float *__restrict__ xo,
+                                                 float *__restrict__ qo)
+{
+    const size_t i = blockIdx.x, row = i * S + S - 1;
+    for (int c = 4 * threadIdx.x; c < D; c += 4 * AT)
+        *(float4 *)(xo + i * D + c) = *(const float4 *)(x + row * D + c);
+    for (int c = 4 * threadIdx.x; c < NQ; c += 4 * AT)
+        *(float4 *)(qo + i * NQ + c) = *(const float4 *)(q + row * NQ + c);
+}
+
+extern "C" int lmk_last_rows(hipStream_t s, const float *x, const float *q, int D, int NQ, int S, int n,
+                             float *xo, float *qo)
+{
+    if (D < 4 || D % 4 || NQ < 4 || NQ % 4 || S < 1 || n < 1 || !x || !q || !xo || !qo)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_last_rows, dim3(n), dim3(AT), 0, s, x, q, D, NQ, S, xo, qo);
+    return hipGetLastError();
+}
+
 /* Work-group count of the 128-query kernel below which the 32-query kernel
  * is used (measured: 24 blocks of 128 (one 256-token prompt, 12 heads) run
  * 1.7x faster split; 192 (eight prompts) 1.3x faster shared). */

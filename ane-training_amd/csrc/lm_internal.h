@@ -174,6 +174,11 @@ int lmk_attn_prefill(hipStream_t s, const float *q, const void *kc, const void *
                      int kv_f32, const int *pos, const int *slot, int S, int nseq,
                      int H, int Hkv, int hd, int max_seq, uint16_t *out);
 
+/* The last row of each of n sequences of S rows: xo[i] = x[i*S + S-1] (D
+ * floats), qo[i] = q[i*S + S-1] (NQ floats).  D and NQ multiples of 4. */
+int lmk_last_rows(hipStream_t s, const float *x, const float *q, int D, int NQ, int S, int n,
+                  float *xo, float *qo);
+
 /* ---- MFMA GEMMs (k_gemm.hip) ----------------------------------------------
  * C[m, n] = sum_k A[m, k] W[n, k], A fp16 [M, lda], W fp16 [N, K], fp32
  * accumulation, on the LDS-tiled MFMA kernel (K % 64 == 0; the tile shape

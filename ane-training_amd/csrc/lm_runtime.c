@@ -892,25 +892,31 @@ static int enqueue_decode_gemv(LMModel *m, int B, float *logits)
  * slot[r]; the K/V of every row is appended to the cache before attention, so
  * rows of one sequence attend causally to each other; seq_rows > 1: the rows
  * are whole sequences of seq_rows rows, attended by the MFMA prefill kernel,
- * else one row per slot, by the decode kernel), then with with_cls the
- * final rmsnorm + classifier of all M rows: logits to `logits` (prefill: only
- * when non-NULL; decode: may be NULL) and, for decode rows, the argmax partials
- * to d_amax. */
+ * else one row per slot, by the decode kernel), then the final rmsnorm +
+ * classifier of the rows: logits to `logits` (decode: may be NULL) and, for
+ * decode rows, the argmax partials to d_amax.  last (prefill, seq_rows > 1):
+ * the logits of each sequence's last row only.  The last layer then owes every
+ * row its K and V but nothing after them: once QKV has run, the last rows'
+ * q and residual are gathered (k_last_rows), attended by the decode kernel,
+ * and only they go on through Wo, the FFN and the classifier; their positions
+ * and slots are in lpos and lslot. */
 static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const int *pos,
-                        const int *slot, float *logits, int with_cls)
+                        const int *slot, float *logits, const int *lpos, const int *lslot)
 {
     hipStream_t s = m->stream;
     const int D = m->D, F = m->F, NQ = m->NQ, NKV = m->NKV, NQKV = NQ + 2 * NKV;
-    const size_t sx = (size_t)M * D;   /* split stride of a [M, D] partial */
+    const int last = lpos != NULL;
+    float *x = m->d_x;
+    size_t sx = (size_t)M * D;   /* split stride of a [M, D] partial */
     /* Wo and W2 write their product, not x: into d_part as fp32 (decode rows
      * (M <= 64) run these narrow projections K-split, one partial per split),
      * and the row norm that next reads x adds it (the residual add).  Only
      * unsplit decode rows keep the residual add in the GEMM epilogue. */
-    const int dec = M <= 64;
+    int dec = M <= 64;
     const int ns_qkv = dec && seq_rows == 1 ? lmk_pick_split(M, NQKV, D) : 1;
-    const int ns_wo = lmk_pick_split(M, D, NQ);
-    const int ns_w2 = lmk_pick_split(M, D, F);
-    const int sep_wo = !dec || ns_wo > 1, sep_w2 = !dec || ns_w2 > 1;
+    int ns_wo = lmk_pick_split(M, D, NQ);
+    int ns_w2 = lmk_pick_split(M, D, F);
+    int sep_wo = !dec || ns_wo > 1, sep_w2 = !dec || ns_w2 > 1;
     /* Beyond 64 rows, an unsplit Wo or W2 folds the row norm that follows it
      * into the GEMMs: it adds its product to x and writes u = fp16(x * gain)
      * and the sums of squares of x per 32 columns (RESNORM), and the GEMM that
@@ -923,9 +929,8 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
      * (LM_OPT_PREFILL_FOLD): u is rounded to fp16 before the row is
      * normalised, and a prefill chunk whose u overflows is redone with the
      * row norm apart (run_prefill); decode rows have no such retry. */
-    const int can_fold = !dec && seq_rows > 1 && m->prefill_fold && !m->fold_off && D % 128 == 0 &&
-                         D / 32 <= 64;
-    const int fold_wo = can_fold && ns_wo == 1, fold_w2 = can_fold && ns_w2 == 1;
+    const int may_fold = seq_rows > 1 && m->prefill_fold && !m->fold_off && D % 128 == 0 && D / 32 <= 64;
+    int fold_wo = may_fold && !dec && ns_wo == 1, fold_w2 = may_fold && !dec && ns_w2 == 1;
     int rs_next = 0;                   /* x's norm is pending in u for QKV */
     const float *pend = NULL;          /* W2 partials not yet added to x */
     int pend_ns = 0;
@@ -959,6 +964,24 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
             KCHK(lmk_gemm(s, m->d_xn16, D, lw, M, NQKV, D, LMK_EPI_QKV, &ep));
         }
         if (ns_qkv > 1) {
+        } else if (last && l == m->L - 1) {
+            /* from here on the sequences' last rows alone, in d_attn (which
+             * holds no prefill rows otherwise): residual, then q */
+            const int n = M / seq_rows;
+            x = m->d_attn;
+            float *lq = x + (size_t)n * D;
+            KCHK(lmk_last_rows(s, m->d_x, m->d_q, D, NQ, seq_rows, n, x, lq));
+            M = n;
+            sx = (size_t)M * D;
+            dec = M <= 64;
+            ns_wo = lmk_pick_split(M, D, NQ);
+            ns_w2 = lmk_pick_split(M, D, F);
+            sep_wo = !dec || ns_wo > 1;
+            sep_w2 = !dec || ns_w2 > 1;
+            fold_wo = may_fold && !dec && ns_wo == 1;
+            fold_w2 = may_fold && !dec && ns_w2 == 1;
+            KCHK(lmk_attn_decode(s, lq, kc, vc, m->kv_f32, lpos, lslot, M, m->H, m->Hkv, m->hd,
+                                 m->max_seq, NULL, m->d_a16));
         } else if (seq_rows > 1) {
             KCHK(lmk_attn_prefill(s, m->d_q, kc, vc, m->kv_f32, pos, slot, seq_rows,
                                   M / seq_rows, m->H, m->Hkv, m->hd, m->max_seq, m->d_a16));
@@ -968,7 +991,7 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
         }
         if (fold_wo) {
             memset(&ep, 0, sizeof(ep));
-            ep.out = m->d_x; ep.ldc = D;
+            ep.out = x; ep.ldc = D;
             ep.gain = m->d_rms_ffn + (size_t)l * D; ep.u = m->d_xn16; ep.ss = m->d_ss; ep.nss = D / 32;
             ep.ovf = m->d_ovf;
             KCHK(lmk_gemm(s, m->d_a16, NQ, lw + m->off_wo, M, D, NQ, LMK_EPI_RESNORM, &ep));
@@ -980,13 +1003,13 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
                 ep.out = m->d_part; ep.ldc = D;
                 KCHK(lmk_gemm(s, m->d_a16, NQ, lw + m->off_wo, M, D, NQ, LMK_EPI_STORE, &ep));
             }
-            KCHK(lmk_rownorm(s, m->d_x, D, M, NULL, NULL, m->d_part, ns_wo, sx,
+            KCHK(lmk_rownorm(s, x, D, M, NULL, NULL, m->d_part, ns_wo, sx,
                              m->d_rms_ffn + (size_t)l * D, m->d_xn16));
         } else {
             memset(&ep, 0, sizeof(ep));
-            ep.out = m->d_x; ep.ldc = D;
+            ep.out = x; ep.ldc = D;
             KCHK(lmk_gemm(s, m->d_a16, NQ, lw + m->off_wo, M, D, NQ, LMK_EPI_RESID, &ep));
-            KCHK(lmk_rownorm(s, m->d_x, D, M, NULL, NULL, NULL, 0, 0,
+            KCHK(lmk_rownorm(s, x, D, M, NULL, NULL, NULL, 0, 0,
                              m->d_rms_ffn + (size_t)l * D, m->d_xn16));
         }
         memset(&ep, 0, sizeof(ep));
@@ -996,7 +1019,7 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
         rs_next = fold_w2 && l + 1 < m->L;
         if (fold_w2) {
             memset(&ep, 0, sizeof(ep));
-            ep.out = m->d_x; ep.ldc = D;
+            ep.out = x; ep.ldc = D;
             if (l + 1 < m->L) {   /* u of the next layer's attention norm */
                 ep.gain = m->d_rms_att + (size_t)(l + 1) * D; ep.u = m->d_xn16; ep.ss = m->d_ss;
                 ep.nss = D / 32; ep.ovf = m->d_ovf;
@@ -1015,22 +1038,15 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
             pend_ns = ns_w2;
         } else {
             memset(&ep, 0, sizeof(ep));
-            ep.out = m->d_x; ep.ldc = D;
+            ep.out = x; ep.ldc = D;
             KCHK(lmk_gemm(s, m->d_g16, F, lw + m->off_w2, M, D, F, LMK_EPI_RESID, &ep));
         }
     }
-    if (!with_cls) {
-        /* x must hold the final residual for the caller: add pending partials */
-        if (pend_ns)
-            KCHK(lmk_rownorm(s, m->d_x, D, M, NULL, NULL, pend, pend_ns, sx, m->d_rms_final,
-                             m->d_xn16));
-        return LM_OK;
-    }
-    KCHK(lmk_rownorm(s, m->d_x, D, M, NULL, NULL, pend, pend_ns, sx, m->d_rms_final, m->d_xn16));
+    KCHK(lmk_rownorm(s, x, D, M, NULL, NULL, pend, pend_ns, sx, m->d_rms_final, m->d_xn16));
     memset(&ep, 0, sizeof(ep));
     ep.out = logits; ep.ldc = m->V; ep.stream_out = 1;
     if (seq_rows > 1) {   /* prefill: logits only */
-        if (logits) KCHK(lmk_gemm(s, m->d_xn16, D, m->d_wcls, M, m->V, D, LMK_EPI_STORE, &ep));
+        KCHK(lmk_gemm(s, m->d_xn16, D, m->d_wcls, M, m->V, D, LMK_EPI_STORE, &ep));
     } else {              /* decode: argmax partials for the greedy step (+ logits) */
         ep.part = m->d_amax;
         KCHK(lmk_gemm(s, m->d_xn16, D, m->d_wcls, M, m->V, D, LMK_EPI_ARGMAX, &ep));
@@ -1041,7 +1057,7 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
 /* One greedy decode step of rows 0..B-1 on the MFMA path (slot b = row b). */
 static int enqueue_decode_gemm(LMModel *m, int B, float *logits)
 {
-    int rc = enqueue_rows(m, B, 1, m->d_tok, m->d_pos, m->d_slot_id, logits, 1);
+    int rc = enqueue_rows(m, B, 1, m->d_tok, m->d_pos, m->d_slot_id, logits, NULL, NULL);
     if (rc) return rc;
     KCHK(lmk_argmax_final(m->stream, m->d_amax, m->cls_nblk, B, m->d_tok, m->d_pos, m->d_hist,
                           m->max_seq + 1, NULL));
@@ -1246,19 +1262,6 @@ int lm_generate_greedy(LMModel *m, int B, const int *first_tokens, const int *po
     return LM_OK;
 }
 
-/* Final rmsnorm + classifier of M rows held in x_rows (fp32 [M, D]): logits to
- * d_logits. */
-static int enqueue_cls_rows(LMModel *m, float *x_rows, int M)
-{
-    hipStream_t s = m->stream;
-    LMEpilogue ep;
-    KCHK(lmk_rownorm(s, x_rows, m->D, M, NULL, NULL, NULL, 0, 0, m->d_rms_final, m->d_xn16));
-    memset(&ep, 0, sizeof(ep));
-    ep.out = m->d_logits; ep.ldc = m->V; ep.stream_out = 1;
-    KCHK(lmk_gemm(s, m->d_xn16, m->D, m->d_wcls, M, m->V, m->D, LMK_EPI_STORE, &ep));
-    return LM_OK;
-}
-
 /* Causal forward of nseq sequences of S tokens (sequence i: slot slots[i],
  * positions pos0[i] .. pos0[i]+S-1, positions below pos0[i] already cached)
  * on the MFMA path, in chunks of whole sequences.  logits_mode LM_LOGITS_ALL:
@@ -1266,14 +1269,16 @@ static int enqueue_cls_rows(LMModel *m, float *x_rows, int M)
  * `logits` (may be NULL) receives them in sequence order; the last chunk's
  * logits stay in d_logits. */
 /* The layers of a prefill chunk of R rows (sequences of S rows; tokens,
- * positions and slots in d_rin, R ints each) and, with `all`, the
- * classifier into d_logits: replayed from a captured graph of that shape
- * (captured on first use) unless graphs are off. */
+ * positions and slots in d_rin, R ints each) and the classifier into d_logits,
+ * of every row with `all`, else of each sequence's last row (positions and
+ * slots after the rows', R/S ints each): replayed from a captured graph of
+ * that shape (captured on first use) unless graphs are off. */
 static int run_rows(LMModel *m, int R, int S, int all)
 {
     const int *tok = m->d_rin, *pos = m->d_rin + R, *slot = m->d_rin + 2 * (size_t)R;
+    const int *lpos = all ? NULL : m->d_rin + 3 * (size_t)R, *lslot = all ? NULL : lpos + R / S;
     if (!m->use_graph || m->fold_off)   /* (the graphs hold the folded form) */
-        return enqueue_rows(m, R, S, tok, pos, slot, all ? m->d_logits : NULL, all);
+        return enqueue_rows(m, R, S, tok, pos, slot, m->d_logits, lpos, lslot);
     int k = 0;
     while (k < PREFILL_GRAPHS &&
            !(m->pgraph[k].ge && m->pgraph[k].R == R && m->pgraph[k].S == S && m->pgraph[k].all == all))
@@ -1287,7 +1292,7 @@ static int run_rows(LMModel *m, int R, int S, int all)
         }
         hipGraph_t g;
         HIPCHK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-        const int rc = enqueue_rows(m, R, S, tok, pos, slot, all ? m->d_logits : NULL, all);
+        const int rc = enqueue_rows(m, R, S, tok, pos, slot, m->d_logits, lpos, lslot);
         hipError_t e = hipStreamEndCapture(m->stream, &g);
         if (rc) return rc;
         HIPCHK(e);
@@ -1348,7 +1353,14 @@ static int run_prefill(LMModel *m, int nseq, const int *slots, const int *pos0, 
                 h[R + r] = pos0[i0 + i] + t;
                 h[2 * R + r] = slots[i0 + i];
             }
-        if (hipMemcpyAsync(m->d_rin, h, (size_t)3 * R * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess) {
+        const int all = logits_mode == LM_LOGITS_ALL || S == 1;   /* (one row: the last) */
+        size_t nin = 3 * (size_t)R;
+        if (!all)
+            for (int i = 0; i < n; i++, nin += 2) {   /* (2n <= R: S >= 2) */
+                h[3 * (size_t)R + i] = pos0[i0 + i] + S - 1;
+                h[3 * (size_t)R + n + i] = slots[i0 + i];
+            }
+        if (hipMemcpyAsync(m->d_rin, h, nin * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess) {
             rc = LM_ERR_HIP;
             break;
         }
@@ -1356,7 +1368,7 @@ static int run_prefill(LMModel *m, int nseq, const int *slots, const int *pos0, 
          * x * gain before the row is normalised): the same rows again with
          * the row norm apart, rewriting the same cache entries */
         for (int pass = 0; pass < 2 && rc == LM_OK; pass++) {
-            if (logits_mode == LM_LOGITS_ALL) {
+            if (all) {
                 rc = run_rows(m, R, S, 1);
                 if (rc == LM_OK && logits &&
                     hipMemcpyAsync(logits + (size_t)i0 * S * V, m->d_logits, (size_t)R * V * 4,
@@ -1372,13 +1384,6 @@ static int run_prefill(LMModel *m, int nseq, const int *slots, const int *pos0, 
                 }
             } else {
                 rc = run_rows(m, R, S, 0);
-                /* gather the last row of each sequence into d_attn (same row width) */
-                if (rc == LM_OK &&
-                    hipMemcpy2DAsync(m->d_attn, (size_t)m->D * 4, m->d_x + (size_t)(S - 1) * m->D,
-                                     (size_t)S * m->D * 4, (size_t)m->D * 4, n,
-                                     hipMemcpyDeviceToDevice, m->stream) != hipSuccess)
-                    rc = LM_ERR_HIP;
-                if (rc == LM_OK) rc = enqueue_cls_rows(m, m->d_attn, n);
                 if (rc == LM_OK && logits &&
                     hipMemcpyAsync(logits + (size_t)i0 * V, m->d_logits, (size_t)n * V * 4,
                                    hipMemcpyDeviceToHost, m->stream) != hipSuccess)
