@@ -255,6 +255,25 @@ int lmk_gemm_split(hipStream_t s, const uint16_t *A, int lda, const uint16_t *W,
 int lmk_rownorm(hipStream_t s, float *x, int D, int M, const uint16_t *emb, const int *tok,
                 const float *sp, int ns, size_t sstride, const float *gain, uint16_t *xn);
 
+/* ---- projections of up to 64 rows (k_rows.hip) ------------------------------
+ * Each with its norm, rotation, residual or gate in one launch; M <= 64, D one
+ * of the model widths, K also 5632 for lmk_rows_res. */
+
+/* Rows m < M: xn = rmsnorm(x[m]) * gain, with emb of the embedding row
+ * emb[tok[m]], which x[m] is set to; [Wq; Wk; Wv] xn, q and k RoPE'd at pos[m];
+ * q to q[m, :NQ], k and v to the cache at (slot[m], pos[m]). */
+int lmk_rows_qkv(hipStream_t s, float *x, const uint16_t *emb, const int *tok, const float *gain,
+                 const uint16_t *wqkv, int D, int M, int NQ, int NKV, int hd, const float *rope_cos,
+                 const float *rope_sin, const int *pos, const int *slot, float *q, void *kc, void *vc,
+                 int kv_f32, int max_seq);
+
+/* x[m, n] += W[n, :K] . a16[m, :K], n < D. */
+int lmk_rows_res(hipStream_t s, const uint16_t *a16, const uint16_t *W, int D, int K, int M, float *x);
+
+/* g[m, i] = fp16(silu(W1[i] . xn) * (W3[i] . xn)), xn = rmsnorm(x[m]) * gain. */
+int lmk_rows_gate(hipStream_t s, const float *x, const float *gain, const uint16_t *w13, int D, int F,
+                  int M, uint16_t *g);
+
 /* ---- loss terms (k_loss.hip) ---------------------------------------------- */
 
 /* M logit rows [M, V] of M/S sequences of S rows, tokens tok[M]: lp[r] =

@@ -888,6 +888,13 @@ static int enqueue_decode_gemv(LMModel *m, int B, float *logits)
 /* Rows per prefill chunk (whole sequences). */
 #define PREFILL_ROWS 2048
 
+/* Whether M rows take the fused projections of k_rows.hip: up to 64 rows of
+ * models up to 1024 wide.  Each work-group there reads its 16 rows whole, which
+ * at width 2048 (131 KB of x beside 64 KB of weights) costs more than the
+ * launches it saves: QKV + gate 10.3 + 13.0 us at 12 rows against 3.7 + 8.4 +
+ * 3.7 + 12.5 for the row norms and tiled GEMMs, W2 (K 5632) 12.5 against 6. */
+static int rows_fused(const LMModel *m, int M) { return M <= 64 && m->D <= 1024 && m->F <= 2048; }
+
 /* Queue the layers for M rows (row r: token tok[r], position pos[r], cache slot
  * slot[r]; the K/V of every row is appended to the cache before attention, so
  * rows of one sequence attend causally to each other; seq_rows > 1: the rows
@@ -934,18 +941,24 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
     int rs_next = 0;                   /* x's norm is pending in u for QKV */
     const float *pend = NULL;          /* W2 partials not yet added to x */
     int pend_ns = 0;
+    int fused = rows_fused(m, M);      /* (also once the last rows are alone) */
     LMEpilogue ep;
     for (int l = 0; l < m->L; l++) {
         const uint16_t *lw = m->d_layers + (size_t)l * m->layer_elems;
         const size_t kvo = (size_t)l * m->kv_layer_elems * (m->kv_f32 ? 4 : 2);
         void *kc = (char *)m->d_kc + kvo, *vc = (char *)m->d_vc + kvo;
         const float *rs = rs_next ? m->d_ss : NULL;   /* u's row scale */
-        if (!rs)
+        if (!rs && !fused)
             KCHK(lmk_rownorm(s, m->d_x, D, M, l == 0 ? m->d_embed : NULL, tok, pend, pend_ns, sx,
                              m->d_rms_att + (size_t)l * D, m->d_xn16));
         pend = NULL;
         pend_ns = 0;
-        if (ns_qkv > 1) {
+        const int split_qkv = ns_qkv > 1 && !fused;
+        if (fused) {
+            KCHK(lmk_rows_qkv(s, x, l == 0 ? m->d_embed : NULL, tok, m->d_rms_att + (size_t)l * D, lw, D,
+                              M, NQ, NKV, m->hd, m->d_rope_cos, m->d_rope_sin, pos, slot, m->d_q, kc, vc,
+                              m->kv_f32, m->max_seq));
+        } else if (split_qkv) {
             /* decode rows, too few column tiles to fill the CUs: K-split QKV;
              * the attention kernel sums the partials, applies RoPE and appends
              * K/V itself */
@@ -963,7 +976,7 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
             ep.rs_ss = rs; ep.nss = D / 32;
             KCHK(lmk_gemm(s, m->d_xn16, D, lw, M, NQKV, D, LMK_EPI_QKV, &ep));
         }
-        if (ns_qkv > 1) {
+        if (split_qkv) {
         } else if (last && l == m->L - 1) {
             /* from here on the sequences' last rows alone, in d_attn (which
              * holds no prefill rows otherwise): residual, then q */
@@ -974,6 +987,7 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
             M = n;
             sx = (size_t)M * D;
             dec = M <= 64;
+            fused = rows_fused(m, M);
             ns_wo = lmk_pick_split(M, D, NQ);
             ns_w2 = lmk_pick_split(M, D, F);
             sep_wo = !dec || ns_wo > 1;
@@ -988,6 +1002,12 @@ static int enqueue_rows(LMModel *m, int M, int seq_rows, const int *tok, const i
         } else {
             KCHK(lmk_attn_decode(s, m->d_q, kc, vc, m->kv_f32, pos, slot, M, m->H, m->Hkv, m->hd,
                                  m->max_seq, NULL, m->d_a16));
+        }
+        if (fused) {   /* the rest of the layer in three launches */
+            KCHK(lmk_rows_res(s, m->d_a16, lw + m->off_wo, D, NQ, M, x));
+            KCHK(lmk_rows_gate(s, x, m->d_rms_ffn + (size_t)l * D, lw + m->off_w13, D, F, M, m->d_g16));
+            KCHK(lmk_rows_res(s, m->d_g16, lw + m->off_w2, D, F, M, x));
+            continue;
         }
         if (fold_wo) {
             memset(&ep, 0, sizeof(ep));
