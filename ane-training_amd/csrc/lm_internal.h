@@ -274,6 +274,32 @@ int lmk_rows_res(hipStream_t s, const uint16_t *a16, const uint16_t *W, int D, i
 int lmk_rows_gate(hipStream_t s, const float *x, const float *gain, const uint16_t *w13, int D, int F,
                   int M, uint16_t *g);
 
+/* ---- the host boundary (k_io.hip) -------------------------------------------
+ * Call block (pinned, read by the device): [0] the call's number, then tokens
+ * and positions of up to LM_CALL_ROWS rows.  Header (pinned, written by the
+ * device): flags and ids.  One flag word per work-group of a give kernel, on a
+ * line of its own, takes the call's number when that work-group's share has
+ * landed; share w of n elements: [w, w + 1) * LM_GIVE_PER(n, work-groups). */
+#define LM_CALL_ROWS 64
+#define LM_CALL_TOK 16
+#define LM_CALL_POS (LM_CALL_TOK + LM_CALL_ROWS)
+#define LM_CALL_INTS (LM_CALL_POS + LM_CALL_ROWS)
+#define LM_HDR_ERR 0
+#define LM_HDR_OVF 1
+#define LM_HDR_TOK 2
+#define LM_HDR_INTS (LM_HDR_TOK + LM_CALL_ROWS)
+#define LM_GIVE_WGS 128
+#define LM_FLAG_STRIDE 16
+#define LM_GIVE_PER(n, wgs) ((((size_t)(n) + (wgs) - 1) / (wgs) + 3) & ~(size_t)3)
+
+int lmk_step_in(hipStream_t s, const int *call, int *seq, int *tok, int *pos, int B);
+int lmk_rows_in(hipStream_t s, const int *h, int *d, int n);
+/* The call's number: *seqp (device), or seqv when seqp is NULL. */
+int lmk_give(hipStream_t s, const float *src, float *dst, size_t n, int wgs, const int *err,
+             const int *ovf, const int *tok, int B, int *hdr, const int *seqp, int seqv, int *flags);
+int lmk_give_ids(hipStream_t s, const int *hist, int stride, const int *pos, int B, int n, int t0, int nt,
+                 int *out, int wgs, const int *err, int *hdr, int seqv, int *flags);
+
 /* ---- loss terms (k_loss.hip) ---------------------------------------------- */
 
 /* M logit rows [M, V] of M/S sequences of S rows, tokens tok[M]: lp[r] =

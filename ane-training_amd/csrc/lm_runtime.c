@@ -19,7 +19,9 @@
  */
 #include "lm_internal.h"
 
+#include <omp.h>
 #include <pthread.h>
+#include <sched.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -36,6 +38,11 @@
 
 #define MAX_GEMV_B 4
 #define PREFILL_GRAPHS 4   /* prefill chunk shapes kept captured */
+#define GIVE_MIN_FLOATS ((size_t)1 << 20)   /* least staging of results: two 2 MiB segments */
+/* What a queued decode step takes in and gives back: a call's step with its
+ * logits or with the ids alone, and the steps of a greedy run (one, or
+ * GRAPH_STEPS), whose inputs and ids the run moves itself. */
+enum { STEP_LOGITS, STEP_IDS, STEP_GREEDY, STEP_GREEDY_N, STEP_KINDS };
 #define CTX_CLASSES 4      /* context lengths the decode attention is launched for (ctx_class) */
 
 struct LMModel {
@@ -67,6 +74,7 @@ struct LMModel {
                                  * (R ints each, back to back), copied in one piece;
                                  * then R floats of loss terms (lm_prefill_loss)     */
     int *h_rin;                 /* their pinned host staging (same layout)          */
+    int *dh_rin;                /* its device address                               */
     /* per-slot greedy state */
     int *d_tok, *d_pos, *d_hist, *d_slot_id;
     /* batch 1-4 chain: QKV, attention (fuse_qa >= 1), Wo (>= 2) and the FFN
@@ -83,12 +91,18 @@ struct LMModel {
     unsigned long long *d_cls_tw;     /* the classifier's argmax partials as tagged words (level 3) */
     unsigned *d_epoch;
     int *d_err;
-    /* pinned host staging */
-    float *h_logits;
-    int *h_io;
-    /* captured decode graphs: [B][0] one step, [B][1] GRAPH_STEPS steps
-     * (greedy feedback stays on the device) */
-    hipGraphExec_t (*step_graph)[2][CTX_CLASSES];   /* [max_batch + 1][2][context class] */
+    /* pinned host staging: results (give_floats floats, at least max_batch
+     * rows of logits); the call block, the header and the flags of k_io.hip
+     * in one block, with their device addresses */
+    float *h_logits, *dh_logits;
+    size_t give_floats;
+    int *h_io;                  /* (lm_profile_chain) and RESNORM's overflow flag */
+    int *h_call, *h_hdr, *h_flag, *dh_call, *dh_hdr, *dh_flag;
+    int *d_seq;                 /* number of the call whose step is running */
+    int seq;
+    /* captured decode graphs by kind of step (greedy feedback stays on the
+     * device) and context class: [max_batch + 1][kind][class] */
+    hipGraphExec_t (*step_graph)[STEP_KINDS][CTX_CLASSES];
     /* captured prefill chunks (the layers and, with all logits, the
      * classifier), by rows, rows per sequence and logits mode; replaced round
      * robin */
@@ -195,6 +209,17 @@ static int dev_alloc(void **p, size_t bytes)
         return LM_ERR_OOM;
     }
     return LM_OK;
+}
+
+/* Pinned host memory and its device address. */
+static int host_alloc(void **h, void **d, size_t bytes)
+{
+    if (hipHostMalloc(h, bytes, 0) != hipSuccess) {
+        fprintf(stderr, "stories_lm: hipHostMalloc(%zu) failed\n", bytes);
+        *h = NULL;
+        return LM_ERR_OOM;
+    }
+    return hipHostGetDevicePointer(d, *h, 0) == hipSuccess ? LM_OK : LM_ERR_HIP;
 }
 
 /* Copy n elements of tensor src (fp32 or fp16) as fp16 into dst (host). */
@@ -330,7 +355,7 @@ static void drop_graphs(LMModel *m)
         }
     if (!m->step_graph) return;
     for (int b = 0; b <= m->max_batch; b++)
-        for (int k = 0; k < 2 * CTX_CLASSES; k++) {
+        for (int k = 0; k < STEP_KINDS * CTX_CLASSES; k++) {
             hipGraphExec_t *ge = &m->step_graph[b][k / CTX_CLASSES][k % CTX_CLASSES];
             if (*ge) {
                 hipGraphExecDestroy(*ge);
@@ -349,7 +374,7 @@ static void free_rows(LMModel *m)
     m->d_x = m->d_q = m->d_attn = m->d_g = m->d_logits = m->d_ss = m->d_part = NULL;
     m->d_g16 = m->d_xn16 = m->d_a16 = NULL;
     m->d_amax = NULL;
-    m->d_rin = m->h_rin = NULL;
+    m->d_rin = m->h_rin = m->dh_rin = NULL;
     m->max_rows = 0;
 }
 
@@ -384,10 +409,7 @@ static int alloc_rows(LMModel *m, int R)
     if ((st = dev_alloc((void **)&m->d_amax, r * m->cls_nblk * sizeof(LMArgPart)))) return st;
     /* tokens, positions and slots of a chunk's rows, then its rows' loss terms */
     if ((st = dev_alloc((void **)&m->d_rin, 4 * r * 4))) return st;
-    if (hipHostMalloc((void **)&m->h_rin, 4 * r * 4, 0) != hipSuccess) {
-        m->h_rin = NULL;
-        return LM_ERR_OOM;
-    }
+    if ((st = host_alloc((void **)&m->h_rin, (void **)&m->dh_rin, 4 * r * 4))) return st;
     m->max_rows = R;
     return LM_OK;
 }
@@ -496,7 +518,7 @@ static LMModel *create_model(const Config *cfg, const WSrc *w, int max_batch, in
     m->layer_elems = m->off_w2 + D * F;
     m->kv_layer_elems = (size_t)max_batch * m->Hkv * max_seq * m->hd;
     const size_t NB = (size_t)max_batch;
-    m->step_graph = (hipGraphExec_t(*)[2][CTX_CLASSES])calloc(NB + 1, sizeof(*m->step_graph));
+    m->step_graph = (hipGraphExec_t(*)[STEP_KINDS][CTX_CLASSES])calloc(NB + 1, sizeof(*m->step_graph));
     if (!m->step_graph) FAIL(LM_ERR_OOM);
 
     if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) FAIL(LM_ERR_HIP);
@@ -537,7 +559,18 @@ static LMModel *create_model(const Config *cfg, const WSrc *w, int max_batch, in
     m->fuse_qa = 3;
     m->layer_wgs = 2;
     m->prefill_fold = 1;
-    if (hipHostMalloc((void **)&m->h_logits, (size_t)max_batch * V * 4, 0) != hipSuccess) FAIL(LM_ERR_OOM);
+    m->give_floats = NB * V > GIVE_MIN_FLOATS ? NB * V : GIVE_MIN_FLOATS;
+    if ((st = host_alloc((void **)&m->h_logits, (void **)&m->dh_logits, m->give_floats * 4))) goto fail;
+    {
+        const size_t nflag = (size_t)2 * LM_GIVE_WGS * LM_FLAG_STRIDE, nint = LM_CALL_INTS + LM_HDR_INTS + 32;
+        if ((st = host_alloc((void **)&m->h_flag, (void **)&m->dh_flag, (nflag + nint) * 4))) goto fail;
+        memset(m->h_flag, 0, (nflag + nint) * 4);
+        m->h_call = m->h_flag + nflag;
+        m->dh_call = m->dh_flag + nflag;
+        m->h_hdr = m->h_call + (LM_CALL_INTS + 15) / 16 * 16;
+        m->dh_hdr = m->dh_call + (LM_CALL_INTS + 15) / 16 * 16;
+    }
+    if ((st = dev_alloc((void **)&m->d_seq, 4))) goto fail;
     if (hipHostMalloc((void **)&m->h_io, (size_t)4 * (max_batch + 1) * 4, 0) != hipSuccess) FAIL(LM_ERR_OOM);
     memset(m->h_io, 0, (size_t)4 * (max_batch + 1) * 4);
     /* RESNORM's overflow flag: the int after the hand-off flag's slot, written
@@ -676,11 +709,12 @@ void lm_free(LMModel *m)
     void *dev[] = {m->d_layers, m->d_embed, m->untied ? m->d_wcls : NULL, m->d_rms_att,
                    m->d_rms_ffn, m->d_rms_final, m->d_rope_cos, m->d_rope_sin, m->d_kc,
                    m->d_vc, m->d_tok, m->d_pos, m->d_hist, m->d_slot_id, m->d_tagged, m->d_cls_tw, m->d_epoch,
-                   m->d_err};
+                   m->d_err, m->d_seq};
     for (size_t i = 0; i < sizeof(dev) / sizeof(dev[0]); i++)
         if (dev[i]) hipFree(dev[i]);
     if (m->h_logits) hipHostFree(m->h_logits);
     if (m->h_io) hipHostFree(m->h_io);
+    if (m->h_flag) hipHostFree(m->h_flag);
     if (m->ev0) hipEventDestroy(m->ev0);
     if (m->ev1) hipEventDestroy(m->ev1);
     if (m->ev_hand) hipEventDestroy(m->ev_hand);
@@ -1092,25 +1126,40 @@ static int enqueue_decode(LMModel *m, int B, float *logits)
 /* Greedy steps captured per multi-step graph. */
 #define GRAPH_STEPS 16
 
-/* Run `nsteps` (1 or GRAPH_STEPS) decode steps of rows 0..B-1, replaying the
- * captured graph of that shape (captured on first use).  Single steps write
- * the logits to d_logits; multi-step runs only feed the argmax forward. */
-static int enqueue_decode_steps(LMModel *m, int B, int nsteps)
+/* Work-groups that give n floats to the host: 4 KiB each, as many as there
+ * are flags. */
+static int give_wgs(size_t n)
 {
-    if (!m->use_graph) {
-        for (int t = 0; t < nsteps; t++) {
-            int rc = enqueue_decode(m, B, nsteps == 1 ? m->d_logits : NULL);
-            if (rc) return rc;
-        }
-        return LM_OK;
-    }
-    hipGraphExec_t *ge = &m->step_graph[B][nsteps == 1 ? 0 : 1][m->ctx_cls];
+    const size_t w = (n + 1023) / 1024;
+    return w < 1 ? 1 : w > LM_GIVE_WGS ? LM_GIVE_WGS : (int)w;
+}
+
+/* Queue the decode steps of `kind` for rows 0..B-1.  Single steps write the
+ * logits to d_logits; multi-step runs only feed the argmax forward. */
+static int enqueue_kind(LMModel *m, int B, int kind)
+{
+    const int call = kind == STEP_LOGITS || kind == STEP_IDS;
+    const size_t n = kind == STEP_LOGITS ? (size_t)B * m->V : 0;
+    int rc = LM_OK;
+    if (call) KCHK(lmk_step_in(m->stream, m->dh_call, m->d_seq, m->d_tok, m->d_pos, B));
+    for (int t = 0; t < (kind == STEP_GREEDY_N ? GRAPH_STEPS : 1) && rc == LM_OK; t++)
+        rc = enqueue_decode(m, B, kind == STEP_GREEDY_N ? NULL : m->d_logits);
+    if (rc || !call) return rc;
+    KCHK(lmk_give(m->stream, n ? m->d_logits : NULL, m->dh_logits, n, give_wgs(n), m->d_err, NULL, m->d_tok, B,
+                  m->dh_hdr, m->d_seq, 0, m->dh_flag));
+    return LM_OK;
+}
+
+/* Run the decode steps of `kind` of rows 0..B-1, replaying the captured graph
+ * of that shape (captured on first use). */
+static int enqueue_decode_steps(LMModel *m, int B, int kind)
+{
+    if (!m->use_graph) return enqueue_kind(m, B, kind);
+    hipGraphExec_t *ge = &m->step_graph[B][kind][m->ctx_cls];
     if (!*ge) {
         hipGraph_t g;
         HIPCHK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-        int rc = LM_OK;
-        for (int t = 0; t < nsteps && rc == LM_OK; t++)
-            rc = enqueue_decode(m, B, nsteps == 1 ? m->d_logits : NULL);
+        const int rc = enqueue_kind(m, B, kind);
         hipError_t e = hipStreamEndCapture(m->stream, &g);
         if (rc) return rc;
         HIPCHK(e);
@@ -1129,37 +1178,101 @@ static int step_waits(const LMModel *m, int B)
     return B <= MAX_GEMV_B && chain_level(m, B) >= 1;
 }
 
-static int run_decode_steps(LMModel *m, int B, int nsteps, int cls)
+static int run_decode_steps(LMModel *m, int B, int kind, int cls)
 {
     m->ctx_cls = cls;
-    if (B > MAX_GEMM_B) {
-        fprintf(stderr, "stories_lm: decode batch %d > %d not supported\n", B, MAX_GEMM_B);
-        return LM_ERR_UNSUPPORTED;
-    }
-    if (nsteps != 1 && nsteps != GRAPH_STEPS) return LM_ERR_INVALID;
-    if (!step_waits(m, B)) return enqueue_decode_steps(m, B, nsteps);
+    if (!step_waits(m, B)) return enqueue_decode_steps(m, B, kind);
     int rc = handoff_enter(m);
     if (rc) return rc;
-    return handoff_leave(m, enqueue_decode_steps(m, B, nsteps));
+    return handoff_leave(m, enqueue_decode_steps(m, B, kind));
 }
 
-
-/* The hand-off flag of the fused QKV + attention launches: queued to the host
- * with the results of a call, checked once the stream has synchronised. */
-static int *err_slot(LMModel *m) { return m->h_io + 4 * (size_t)m->max_batch; }
-
-static int queue_err_read(LMModel *m)
+static int check_batch(int B)
 {
-    return hipMemcpyAsync(err_slot(m), m->d_err, 4, hipMemcpyDeviceToHost, m->stream) == hipSuccess
-               ? LM_OK
-               : LM_ERR_HIP;
+    if (B <= MAX_GEMM_B) return LM_OK;
+    fprintf(stderr, "stories_lm: decode batch %d > %d not supported\n", B, MAX_GEMM_B);
+    return LM_ERR_UNSUPPORTED;
 }
 
-static int check_err(LMModel *m)
+/* The next call number (never 0 but at a wrap of 2^32; the flags start at 0). */
+static int next_seq(LMModel *m) { return m->seq = (int)((unsigned)m->seq + 1u); }
+
+/* Wait until flag k of set `set` carries `seq`: the share of that work-group
+ * of a give kernel has landed.  Polled, since a stream synchronise returns
+ * about 8 us later; now and then the stream is asked, so that work that ended
+ * without raising the flag (a failed launch) ends the wait as well. */
+static int wait_flag(LMModel *m, int set, int k, int seq)
 {
-    if (!*err_slot(m)) return LM_OK;
+    const int *f = m->h_flag + ((size_t)set * LM_GIVE_WGS + k) * LM_FLAG_STRIDE;
+    for (unsigned spin = 1; __atomic_load_n(f, __ATOMIC_ACQUIRE) != seq; spin++) {
+        __builtin_ia32_pause();
+        if (spin & 4095) continue;
+        const hipError_t e = hipStreamQuery(m->stream);
+        if (e == hipErrorNotReady) {
+            (void)hipGetLastError();   /* (not an error of a launch to come) */
+            sched_yield();
+            continue;
+        }
+        if (e == hipSuccess && __atomic_load_n(f, __ATOMIC_ACQUIRE) == seq) break;
+        fprintf(stderr, "stories_lm: results did not arrive: %s\n", hipGetErrorString(e));
+        return LM_ERR_HIP;
+    }
+    return LM_OK;
+}
+
+/* Copy n floats that a give kernel of `wgs` work-groups stages at src to dst
+ * (NULL: only wait), share by share as they land; from 1 MiB on with up to
+ * four threads (one thread copies 32 MiB to fresh pages in 1.0 ms, four in
+ * 0.2-0.5, while they cross the bus in 0.58). */
+static int take(LMModel *m, int set, int seq, const float *src, float *dst, size_t n, int wgs)
+{
+    const size_t per = LM_GIVE_PER(n, wgs);
+    const int nt = dst && n >= ((size_t)1 << 18) ? (omp_get_max_threads() < 4 ? omp_get_max_threads() : 4) : 1;
+    int rc = LM_OK;
+#pragma omp parallel for num_threads(nt) schedule(static, 1) if (nt > 1)
+    for (int k = 0; k < wgs; k++) {
+        const int st = wait_flag(m, set, k, seq);
+        const size_t a = per * k, e = a + per < n ? a + per : n;
+        if (st) {
+#pragma omp atomic write
+            rc = st;
+        } else if (dst && a < e) {
+            memcpy(dst + a, src + a, (e - a) * 4);
+        }
+    }
+    return rc;
+}
+
+/* n floats of device memory (complete on the stream) to the caller's dst in
+ * segments of half the staging, one crossing the bus while the host copies the
+ * other; the overflow flag of the stream's work comes with them in the header. */
+static int give(LMModel *m, const float *src, float *dst, size_t n)
+{
+    const size_t half = m->give_floats / 2 & ~(size_t)3;
+    const size_t seg = half < ((size_t)1 << 19) ? half : (size_t)1 << 19;
+    const size_t nseg = (n + seg - 1) / seg;
+    int seqs[2] = {0, 0}, rc = LM_OK;
+    for (size_t i = 0; i < nseg + 1 && rc == LM_OK; i++) {
+        if (i < nseg) {   /* segment i into half i & 1, which segment i - 2 has left */
+            const size_t a = i * seg, c = a + seg < n ? seg : n - a;
+            seqs[i & 1] = next_seq(m);
+            KCHK(lmk_give(m->stream, src + a, m->dh_logits + (i & 1) * seg, c, give_wgs(c), NULL, m->d_ovf, NULL, 0,
+                          m->dh_hdr, NULL, seqs[i & 1], m->dh_flag + (i & 1) * LM_GIVE_WGS * LM_FLAG_STRIDE));
+        }
+        if (i > 0) {
+            const size_t j = i - 1, a = j * seg, c = a + seg < n ? seg : n - a;
+            rc = take(m, (int)(j & 1), seqs[j & 1], m->h_logits + (j & 1) * seg, dst + a, c, give_wgs(c));
+        }
+    }
+    return rc;
+}
+
+/* The hand-off flag of the fused launches, as a call's results brought it. */
+static int check_err(LMModel *m, int err)
+{
+    if (!err) return LM_OK;
     fprintf(stderr, "stories_lm: a hand-off wait inside a fused launch gave up (results invalid)\n");
-    *err_slot(m) = 0;
+    HIPCHK(hipStreamSynchronize(m->stream));
     /* Once a wait has given up, every wait of the launch ends early, so the
      * argmax reducer can advance the step count while classifier work-groups
      * dispatched before it have yet to read it; their words then carry the
@@ -1187,28 +1300,32 @@ static int check_tok_pos(const LMModel *m, const int *tokens, const int *pos, in
     return LM_OK;
 }
 
+/* One decode step of a call: its inputs into the call block, the step, its
+ * logits (logits, B x V, may be NULL: staged in h_logits) and header. */
+static int step_call(LMModel *m, const int *tokens, const int *pos, int B, int kind, float *logits)
+{
+    memcpy(m->h_call + LM_CALL_TOK, tokens, (size_t)B * 4);
+    memcpy(m->h_call + LM_CALL_POS, pos, (size_t)B * 4);
+    const int seq = next_seq(m);
+    __atomic_store_n(m->h_call, seq, __ATOMIC_RELEASE);
+    const size_t n = kind == STEP_LOGITS ? (size_t)B * m->V : 0;
+    int rc = run_decode_steps(m, B, kind, ctx_class_rows(pos, B, 0));
+    if (rc == LM_OK) rc = take(m, 0, seq, m->h_logits, logits, n, give_wgs(n));
+    if (rc != LM_OK) {
+        (void)hipStreamSynchronize(m->stream);   /* the call block is free again */
+        return rc;
+    }
+    return check_err(m, m->h_hdr[LM_HDR_ERR]);
+}
+
 int lm_forward_batch(LMModel *m, const int *tokens, const int *pos, int B, float *logits, int *argmax)
 {
     if (!m || !tokens || !pos || B < 1) return LM_ERR_INVALID;
     if (B > m->max_batch) return LM_ERR_RANGE;
     int rc = check_tok_pos(m, tokens, pos, B);
-    if (rc) return rc;
-    int *hio = m->h_io;
-    memcpy(hio, tokens, B * 4);
-    memcpy(hio + B, pos, B * 4);
-    HIPCHK(hipMemcpyAsync(m->d_tok, hio, B * 4, hipMemcpyHostToDevice, m->stream));
-    HIPCHK(hipMemcpyAsync(m->d_pos, hio + B, B * 4, hipMemcpyHostToDevice, m->stream));
-    if ((rc = run_decode_steps(m, B, 1, ctx_class_rows(pos, B, 0)))) return rc;
-    if (argmax)
-        HIPCHK(hipMemcpyAsync(hio + 2 * B, m->d_tok, B * 4, hipMemcpyDeviceToHost, m->stream));
-    if (logits)
-        HIPCHK(hipMemcpyAsync(m->h_logits, m->d_logits, (size_t)B * m->V * 4,
-                              hipMemcpyDeviceToHost, m->stream));
-    if ((rc = queue_err_read(m))) return rc;
-    HIPCHK(hipStreamSynchronize(m->stream));
-    if ((rc = check_err(m))) return rc;
-    if (argmax) memcpy(argmax, hio + 2 * B, B * 4);
-    if (logits) memcpy(logits, m->h_logits, (size_t)B * m->V * 4);
+    if (rc || (rc = check_batch(B))) return rc;
+    if ((rc = step_call(m, tokens, pos, B, logits ? STEP_LOGITS : STEP_IDS, logits))) return rc;
+    if (argmax) memcpy(argmax, m->h_hdr + LM_HDR_TOK, (size_t)B * 4);
     return LM_OK;
 }
 
@@ -1219,21 +1336,7 @@ const float *lm_forward(LMModel *m, int token, int pos)
         return NULL;
     }
     if (check_tok_pos(m, &token, &pos, 1)) return NULL;
-    int *hio = m->h_io;
-    hio[0] = token;
-    hio[1] = pos;
-    if (hipMemcpyAsync(m->d_tok, hio, 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
-        hipMemcpyAsync(m->d_pos, hio + 1, 4, hipMemcpyHostToDevice, m->stream) != hipSuccess)
-        return NULL;
-    if (run_decode_steps(m, 1, 1, ctx_class(pos))) return NULL;
-    if (hipMemcpyAsync(m->h_logits, m->d_logits, (size_t)m->V * 4, hipMemcpyDeviceToHost,
-                       m->stream) != hipSuccess ||
-        queue_err_read(m) != LM_OK || hipStreamSynchronize(m->stream) != hipSuccess) {
-        fprintf(stderr, "stories_lm: lm_forward: HIP error\n");
-        return NULL;
-    }
-    if (check_err(m)) return NULL;
-    return m->h_logits;
+    return step_call(m, &token, &pos, 1, STEP_LOGITS, NULL) ? NULL : m->h_logits;
 }
 
 int lm_generate_greedy(LMModel *m, int B, const int *first_tokens, const int *pos0, int n_steps,
@@ -1250,36 +1353,30 @@ int lm_generate_greedy(LMModel *m, int B, const int *first_tokens, const int *po
             return LM_ERR_RANGE;
         }
     if (n_steps == 0) return LM_OK;
-    int *hio = m->h_io;
-    memcpy(hio, first_tokens, B * 4);
-    memcpy(hio + B, pos0, B * 4);
-    HIPCHK(hipMemcpyAsync(m->d_tok, hio, B * 4, hipMemcpyHostToDevice, m->stream));
-    HIPCHK(hipMemcpyAsync(m->d_pos, hio + B, B * 4, hipMemcpyHostToDevice, m->stream));
+    if ((rc = check_batch(B))) return rc;
+    memcpy(m->h_call + LM_CALL_TOK, first_tokens, (size_t)B * 4);
+    memcpy(m->h_call + LM_CALL_POS, pos0, (size_t)B * 4);
+    __atomic_store_n(m->h_call, next_seq(m), __ATOMIC_RELEASE);
+    KCHK(lmk_step_in(m->stream, m->dh_call, m->d_seq, m->d_tok, m->d_pos, B));
     int t = 0;
-    for (; t + GRAPH_STEPS <= n_steps; t += GRAPH_STEPS)
-        if ((rc = run_decode_steps(m, B, GRAPH_STEPS, ctx_class_rows(pos0, B, t + GRAPH_STEPS - 1)))) return rc;
-    for (; t < n_steps; t++)
-        if ((rc = run_decode_steps(m, B, 1, ctx_class_rows(pos0, B, t)))) return rc;
-    const size_t stride = (size_t)m->max_seq + 1;
-    int *h = (int *)malloc((size_t)B * stride * 4);
-    if (!h) return LM_ERR_OOM;
-    hipError_t e = hipMemcpyAsync(h, m->d_hist, (size_t)B * stride * 4, hipMemcpyDeviceToHost, m->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(err_slot(m), m->d_err, 4, hipMemcpyDeviceToHost, m->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-    if (e != hipSuccess) {
-        free(h);
-        fprintf(stderr, "stories_lm: lm_generate_greedy: %s\n", hipGetErrorString(e));
-        return LM_ERR_HIP;
+    for (; t + GRAPH_STEPS <= n_steps && rc == LM_OK; t += GRAPH_STEPS)
+        rc = run_decode_steps(m, B, STEP_GREEDY_N, ctx_class_rows(pos0, B, t + GRAPH_STEPS - 1));
+    for (; t < n_steps && rc == LM_OK; t++)
+        rc = run_decode_steps(m, B, STEP_GREEDY, ctx_class_rows(pos0, B, t));
+    /* the ids, as many steps at a time as the staging holds */
+    const int seg = m->give_floats / B < (size_t)n_steps ? (int)(m->give_floats / B) : n_steps;
+    for (int t0 = 0; t0 < n_steps && rc == LM_OK; t0 += seg) {
+        const int nt = t0 + seg < n_steps ? seg : n_steps - t0, wgs = give_wgs((size_t)nt * B), seq = next_seq(m);
+        if (lmk_give_ids(m->stream, m->d_hist, m->max_seq + 1, m->d_pos, B, n_steps, t0, nt,
+                         (int *)m->dh_logits, wgs, m->d_err, m->dh_hdr, seq, m->dh_flag) != hipSuccess)
+            rc = LM_ERR_HIP;
+        else rc = take(m, 0, seq, m->h_logits, (float *)out_tokens + (size_t)t0 * B, (size_t)nt * B, wgs);
     }
-    if ((rc = check_err(m))) {
-        free(h);
+    if (rc != LM_OK) {
+        (void)hipStreamSynchronize(m->stream);
         return rc;
     }
-    for (int t = 0; t < n_steps; t++)
-        for (int b = 0; b < B; b++) out_tokens[(size_t)t * B + b] = h[b * stride + pos0[b] + 1 + t];
-    free(h);
-    return LM_OK;
+    return check_err(m, m->h_hdr[LM_HDR_ERR]);
 }
 
 /* Causal forward of nseq sequences of S tokens (sequence i: slot slots[i],
@@ -1289,7 +1386,7 @@ int lm_generate_greedy(LMModel *m, int B, const int *first_tokens, const int *po
  * `logits` (may be NULL) receives them in sequence order; the last chunk's
  * logits stay in d_logits. */
 /* The layers of a prefill chunk of R rows (sequences of S rows; tokens,
- * positions and slots in d_rin, R ints each) and the classifier into d_logits,
+ * positions and slots, R ints each, read from h_rin into d_rin) and the classifier into d_logits,
  * of every row with `all`, else of each sequence's last row (positions and
  * slots after the rows', R/S ints each): replayed from a captured graph of
  * that shape (captured on first use) unless graphs are off. */
@@ -1297,8 +1394,11 @@ static int run_rows(LMModel *m, int R, int S, int all)
 {
     const int *tok = m->d_rin, *pos = m->d_rin + R, *slot = m->d_rin + 2 * (size_t)R;
     const int *lpos = all ? NULL : m->d_rin + 3 * (size_t)R, *lslot = all ? NULL : lpos + R / S;
-    if (!m->use_graph || m->fold_off)   /* (the graphs hold the folded form) */
+    const int nin = 3 * R + (all ? 0 : 2 * (R / S));
+    if (!m->use_graph || m->fold_off) {   /* (the graphs hold the folded form) */
+        KCHK(lmk_rows_in(m->stream, m->dh_rin, m->d_rin, nin));
         return enqueue_rows(m, R, S, tok, pos, slot, m->d_logits, lpos, lslot);
+    }
     int k = 0;
     while (k < PREFILL_GRAPHS &&
            !(m->pgraph[k].ge && m->pgraph[k].R == R && m->pgraph[k].S == S && m->pgraph[k].all == all))
@@ -1312,7 +1412,8 @@ static int run_rows(LMModel *m, int R, int S, int all)
         }
         hipGraph_t g;
         HIPCHK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-        const int rc = enqueue_rows(m, R, S, tok, pos, slot, m->d_logits, lpos, lslot);
+        int rc = lmk_rows_in(m->stream, m->dh_rin, m->d_rin, nin) == hipSuccess ? LM_OK : LM_ERR_HIP;
+        if (rc == LM_OK) rc = enqueue_rows(m, R, S, tok, pos, slot, m->d_logits, lpos, lslot);
         hipError_t e = hipStreamEndCapture(m->stream, &g);
         if (rc) return rc;
         HIPCHK(e);
@@ -1361,7 +1462,7 @@ static int run_prefill(LMModel *m, int nseq, const int *slots, const int *pos0, 
     const int chunk_rows = (nseq < cs ? nseq : cs) * S;
     int rc;
     if (chunk_rows > m->max_rows && (rc = alloc_rows(m, chunk_rows))) return rc;
-    int *h = m->h_rin;   /* pinned; each chunk ends with a stream synchronise */
+    int *h = m->h_rin;   /* pinned; each chunk ends with its results at the host */
     rc = LM_OK;
     for (int i0 = 0; i0 < nseq && rc == LM_OK; i0 += cs) {
         const int n = nseq - i0 < cs ? nseq - i0 : cs;
@@ -1374,43 +1475,31 @@ static int run_prefill(LMModel *m, int nseq, const int *slots, const int *pos0, 
                 h[2 * R + r] = slots[i0 + i];
             }
         const int all = logits_mode == LM_LOGITS_ALL || S == 1;   /* (one row: the last) */
-        size_t nin = 3 * (size_t)R;
         if (!all)
-            for (int i = 0; i < n; i++, nin += 2) {   /* (2n <= R: S >= 2) */
+            for (int i = 0; i < n; i++) {   /* (2n <= R: S >= 2) */
                 h[3 * (size_t)R + i] = pos0[i0 + i] + S - 1;
                 h[3 * (size_t)R + n + i] = slots[i0 + i];
             }
-        if (hipMemcpyAsync(m->d_rin, h, nin * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess) {
-            rc = LM_ERR_HIP;
-            break;
-        }
         /* pass 1 only when pass 0's folded norm overflowed fp16 (its u is
          * x * gain before the row is normalised): the same rows again with
          * the row norm apart, rewriting the same cache entries */
         for (int pass = 0; pass < 2 && rc == LM_OK; pass++) {
-            if (all) {
-                rc = run_rows(m, R, S, 1);
-                if (rc == LM_OK && logits &&
-                    hipMemcpyAsync(logits + (size_t)i0 * S * V, m->d_logits, (size_t)R * V * 4,
-                                   hipMemcpyDeviceToHost, m->stream) != hipSuccess)
-                    rc = LM_ERR_HIP;
-                /* the chunk's loss terms, before the next chunk reuses d_logits */
-                if (rc == LM_OK && loss) {
-                    float *d_lp = (float *)(m->d_rin + 3 * (size_t)R);
-                    if (lmk_row_logprob(m->stream, m->d_logits, V, m->d_rin, S, R, d_lp) != hipSuccess ||
-                        hipMemcpyAsync(h + 3 * (size_t)R, d_lp, (size_t)R * 4, hipMemcpyDeviceToHost,
-                                       m->stream) != hipSuccess)
-                        rc = LM_ERR_HIP;
-                }
-            } else {
-                rc = run_rows(m, R, S, 0);
-                if (rc == LM_OK && logits &&
-                    hipMemcpyAsync(logits + (size_t)i0 * V, m->d_logits, (size_t)n * V * 4,
-                                   hipMemcpyDeviceToHost, m->stream) != hipSuccess)
-                    rc = LM_ERR_HIP;
-            }
-            if (rc == LM_OK && hipStreamSynchronize(m->stream) != hipSuccess) rc = LM_ERR_HIP;
+            rc = run_rows(m, R, S, all);
+            /* the chunk's loss terms, straight to the staging, before the next
+             * chunk reuses d_logits */
+            if (rc == LM_OK && loss &&
+                lmk_row_logprob(m->stream, m->d_logits, V, m->d_rin, S, R,
+                                (float *)(m->dh_rin + 3 * (size_t)R)) != hipSuccess)
+                rc = LM_ERR_HIP;
+            const size_t rows = logits_mode == LM_LOGITS_ALL ? (size_t)R : (size_t)n;
+            const size_t row0 = logits_mode == LM_LOGITS_ALL ? (size_t)i0 * S : (size_t)i0;
             volatile int *ovf = m->h_io + 4 * (size_t)m->max_batch + 1;
+            if (rc == LM_OK && logits) {
+                rc = give(m, m->d_logits, logits + row0 * V, rows * V);
+                if (rc == LM_OK) *ovf = m->h_hdr[LM_HDR_OVF];
+            }
+            if (rc == LM_OK && (!logits || loss) && hipStreamSynchronize(m->stream) != hipSuccess)
+                rc = LM_ERR_HIP;
             if (rc != LM_OK || !*ovf) break;
             *ovf = 0;
             m->fold_off = 1;
@@ -1478,6 +1567,7 @@ int lm_read_logits(LMModel *m, int row0, int nrows, float *dst)
 {
     if (!m || !dst || row0 < 0 || nrows < 0) return LM_ERR_INVALID;
     if (row0 + nrows > m->max_rows) return LM_ERR_RANGE;
+    HIPCHK(hipStreamSynchronize(m->stream));
     HIPCHK(hipMemcpy(dst, m->d_logits + (size_t)row0 * m->V, (size_t)nrows * m->V * 4,
                      hipMemcpyDeviceToHost));
     return LM_OK;
@@ -1616,9 +1706,11 @@ int lm_profile_chain(LMModel *m, int B, const int *tokens, const int *pos, int s
     free(kl);
     if (rc == LM_OK)
         HIPCHK(hipMemcpyAsync(m->d_pos, hio + B, B * 4, hipMemcpyHostToDevice, m->stream));
-    if (rc == LM_OK) rc = queue_err_read(m);
+    int *err = hio + 4 * (size_t)m->max_batch;
+    if (rc == LM_OK && hipMemcpyAsync(err, m->d_err, 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess)
+        rc = LM_ERR_HIP;
     HIPCHK(hipStreamSynchronize(m->stream));
-    if (rc == LM_OK) rc = check_err(m);
+    if (rc == LM_OK) rc = check_err(m, *err);
     return rc;
 }
 

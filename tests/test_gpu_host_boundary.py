@@ -1,0 +1,59 @@
+"""Results as kernels give them to the host (shares with a flag each, segments of
+the staging), against the device's own copy of the logits."""
+import numpy as np
+import pytest
+
+from conftest import TINY
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(lm, vocab, B, S):
+    cfg = lm.make_config(**dict(TINY, vocab_size=vocab))
+    return lm.Model.create(cfg, lm.synth_weights_f16(cfg, 97, 0.02, True), True, B, S)
+
+
+@pytest.mark.parametrize("vocab", [1, 3, 301, 1023, 1024, 1025, 40001])
+@pytest.mark.parametrize("B", [1, 2, 7, 64])
+def test_step_results_equal_device_logits(lm, vocab, B):
+    """The same values bit for bit, ids the first maximum; changing inputs, so
+    that a result of the call before would show."""
+    with _model(lm, vocab, B, 16) as m:
+        rng = np.random.default_rng(vocab + B)
+        for p in range(4):
+            tk = rng.integers(0, vocab, B).astype(np.int32)
+            lg, am = m.forward_batch(tk, np.full(B, p, np.int32))
+            assert np.array_equal(lg, m.read_logits(0, B))
+            assert np.array_equal(am, lg.argmax(1))
+            none, am2 = m.forward_batch(tk, np.full(B, p, np.int32), want_logits=False)
+            assert none is None and np.array_equal(am, am2)
+        one = m.forward(int(tk[0]), 3)
+        assert np.array_equal(one, m.read_logits(0, 1)[0])
+
+
+@pytest.mark.parametrize("vocab,n,S", [(301, 3, 5), (32000, 1, 40), (32001, 2, 33), (9001, 5, 47)])
+def test_prompt_logits_equal_device_logits(lm, vocab, n, S):
+    """Several segments (more than 2 MiB), the last ragged, into fresh and
+    reused host memory."""
+    with _model(lm, vocab, n, S) as m:
+        rng = np.random.default_rng(S)
+        for _ in range(3):
+            toks = rng.integers(0, vocab, (n, S)).astype(np.int32)
+            lg = m.prefill_batch(toks, mode=lm.LM_LOGITS_ALL)
+            assert np.array_equal(lg, m.read_logits(0, n * S))
+            loss, lg2 = m.prefill_loss(toks, want_logits=True) if vocab % 4 == 0 else (None, lg)
+            assert np.array_equal(lg, lg2)
+            last = m.prefill_batch(toks, mode=lm.LM_LOGITS_LAST)
+            assert np.array_equal(last, m.read_logits(0, n))
+
+
+@pytest.mark.parametrize("B,steps", [(1, 1), (1, 16), (3, 33), (64, 50)])
+def test_greedy_ids_equal_single_steps(lm, B, steps):
+    """A run of the device loop against its steps one call at a time."""
+    with _model(lm, 2, B, 64) as m:
+        first = (np.arange(B) % 2).astype(np.int32)
+        ids = m.generate_greedy(first, np.zeros(B, np.int32), steps)
+        tk = first
+        for t in range(steps):
+            tk = m.forward_batch(tk, np.full(B, t, np.int32), want_logits=False)[1]
+            assert np.array_equal(ids[t], tk), t
