@@ -24,11 +24,12 @@
  * 16-byte units so that neither the transposing writes nor the fragment reads
  * conflict in the LDS banks.
  *
- * Two work-group shapes share that per-tile step:
- *   k_attn_prefill_blk    128 queries per work-group, 32 per wave; the four
- *                         waves share each staged tile (K/V of tile t+2 in
- *                         registers while tile t computes, tile t+1 in the other
- *                         LDS buffer).  Least K/V traffic: for many blocks.
+ * Two kernels share that per-tile step:
+ *   k_attn_prefill_blk    64 or 128 queries per work-group, 32 per wave; all
+ *                         waves share each staged key tile, and where there are
+ *                         more waves than query groups they take a step's tiles
+ *                         in halves and merge at the end.  Least K/V traffic:
+ *                         for many blocks.
  *   k_attn_prefill_split  32 queries per work-group; the four waves split the
  *                         key tiles round-robin, each staging its own, and merge
  *                         their (m, l, O) through LDS.  The last query block waits
@@ -192,51 +193,79 @@ __device__ __forceinline__ void load_q(const float *q, size_t row, int NQ, int h
     for (int ks = 0; ks < HD / 16; ks++) qb16[ks] = kv8_f16(qs + ks * 16);
 }
 
-/* ---- 128-query blocks, shared tiles ---------------------------------------- */
+/* Head, sequence and query block of work-group id of nqb * nseq * H.  It runs
+ * on XCD id % 8: heads fastest, neighbouring heads (one kv head's) on one XCD
+ * where the count allows, so that an XCD's L2 holds the K and V of few heads;
+ * a prompt's longest blocks first, so that the short ones fill the end. */
+__device__ __forceinline__ void block_of(int id, int nqb, int nseq, int H, int &h, int &seq, int &qb)
+{
+    const int bi = small_div(id, H), hi = id - bi * H;
+    h = H % 8 == 0 ? (hi & 7) * (H >> 3) + (hi >> 3) : hi;
+    const int qr = small_div(bi, nseq);
+    seq = bi - qr * nseq;
+    qb = nqb - 1 - qr;
+}
 
-#define BQB 128         /* query rows per work-group */
+/* ---- 64- and 128-query blocks, shared tiles --------------------------------- */
 
-template <int HD, typename KT>
-__global__ void __launch_bounds__(AT) k_attn_prefill_blk(
+/* W waves, QG of them along the block's queries (32 each), KG = W / QG along its
+ * keys: a step stages KG consecutive key tiles, wave (qg, kg) takes tile kg of
+ * them for the 32 queries of group qg, and with KG = 2 the two halves'
+ * (m, l, O) meet in LDS at the end.  What bounds it is the longest chain of
+ * dependent tiles and each tile's latency (MFMA, exp2, MFMA, barrier): the last
+ * block of a prompt walks all its key tiles.  One 1900-token prompt in
+ * 128-query blocks has fewer work-groups than CUs and lasts as long as 30
+ * tiles in turn; KG 2 halves the chain.  us per launch at 1900: hd 128, 16
+ * heads, four waves of 128 queries 70, eight waves KG 2 53; hd 64, 12 heads, 35.5
+ * against 25.8 with 64-query blocks KG 2. */
+template <int HD, typename KT, int QG, int W>
+__global__ void __launch_bounds__(64 * W, W == 8 || QG == 2 ? 2 : 1) k_attn_prefill_blk(
     const float *__restrict__ q, const KT *__restrict__ kc, const KT *__restrict__ vc,
-    const int *__restrict__ pos, const int *__restrict__ slot, int S, int nqb, int H, int Hkv,
+    const int *__restrict__ pos, const int *__restrict__ slot, int S, int nseq, int nqb, int H, int Hkv,
     int max_seq, u16 *__restrict__ out)
 {
+    constexpr int KG = W / QG, BQ = 32 * QG, NT = 64 * W;
     constexpr int KLD = HD + 8;          /* K tile row stride (halves)   */
     constexpr int DT = HD / 32;          /* 32-dim row tiles of O^T      */
-    constexpr int PPT = BKV * HD / 16 / AT;  /* staging units per thread */
-    static_assert(PPT >= 1 && BKV * HD / 16 % AT == 0, "staging shape");
-    __shared__ __attribute__((aligned(16))) u16 sk[2][BKV * KLD];
-    __shared__ __attribute__((aligned(16))) u16 svt[2][HD * BKV];
+    constexpr int UPT = BKV * HD / 16, PPT = KG * UPT / NT;   /* staging units per tile; per thread and step */
+    constexpr int NB = 2;
+    constexpr int TS = BKV * KLD + HD * BKV;      /* halves of one tile's K and V^T */
+    constexpr int MLD = HD + 1;                   /* merge row stride (floats) */
+    static_assert(PPT >= 1 && KG * UPT % NT == 0 && (UPT % NT == 0 || NT % UPT == 0), "staging shape");
+    static_assert(KG == 1 || NB * KG * TS * 2 >= (QG * 32 * MLD + 2 * QG * 32) * 4, "merge area fits the staging area");
+    __shared__ __attribute__((aligned(16))) u16 stg[NB][KG * TS];
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int seq = small_div(blockIdx.x, nqb), qb = blockIdx.x - seq * nqb;
-    const int h = blockIdx.y;
+    const int qg = wave % QG, kg = wave / QG;
+    int h, seq, qb;
+    block_of(blockIdx.x, nqb, nseq, H, h, seq, qb);
     const int kvh = small_div(h, small_div(H, Hkv));
     const int NQ = H * HD;
-    const int row0 = seq * S + qb * BQB;          /* first row of the block       */
-    const int nrows = min(BQB, S - qb * BQB);     /* valid rows of the block      */
+    const int row0 = seq * S + qb * BQ;           /* first row of the block       */
+    const int nrows = min(BQ, S - qb * BQ);       /* valid rows of the block      */
     const int p0 = pos[row0];                     /* position of the block's row 0 */
     const int cs = slot[row0];
     const size_t cbase = ((size_t)cs * Hkv + kvh) * max_seq * HD;
     /* scores are kept in log2 units: exp(x) = exp2(x * log2 e) */
     const float scale = 1.4426950408889634f / sqrtf((float)HD);
     const int last_pos = p0 + nrows - 1;          /* last query position of the block */
-    const int ntiles = last_pos / BKV + 1;
+    const int nsteps = (last_pos / BKV + KG) / KG;
 
-    /* K / V of one tile: thread t stages units t + i*AT (two keys, 8 dims each:
-     * [0] key, [1] key + 1); keys past the block's last position repeat it (they
-     * are masked for every query that reads them).  Two register sets: tile t
-     * sits in set t % 2 from its fetch (two tiles ahead of its use) until it is
-     * stored to LDS (one tile ahead). */
-    uint4 rk0[PPT][2], rv0[PPT][2], rk1[PPT][2], rv1[PPT][2];
-    auto fetch = [&](int kt, uint4 (&rk)[PPT][2], uint4 (&rv)[PPT][2]) {
+    /* K / V of one step: thread t stages units t + i*AT (two keys, 8 dims each:
+     * [0] key, [1] key + 1; KG = 2: the first half of the units is tile 0's);
+     * keys past the block's last position repeat it (they are masked for every
+     * query that reads them).  Two register sets: step t sits in set t % 2 from
+     * its fetch (two steps ahead of its use) until it is stored to LDS; one
+     * set, one step ahead, at KG 2. */
+    constexpr int NSET = KG == 1 ? 2 : 1;
+    uint4 rk0[PPT][2], rv0[PPT][2], rk1[NSET == 2 ? PPT : 1][2], rv1[NSET == 2 ? PPT : 1][2];
+    auto fetch = [&](int st, auto &rk, auto &rv) {
 #pragma unroll
         for (int i = 0; i < PPT; i++) {
             int pk, d0;
-            pair_of<HD>(tid + i * AT, pk, d0);
-            const int key = kt * BKV + vperm(pk);
+            pair_of<HD>((tid + i * NT) % UPT, pk, d0);
+            const int key = (st * KG + (tid + i * NT) / UPT) * BKV + vperm(pk);
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 const size_t off = cbase + (size_t)min(key + e, last_pos) * HD + d0;
@@ -245,19 +274,20 @@ __global__ void __launch_bounds__(AT) k_attn_prefill_blk(
             }
         }
     };
-    auto stash = [&](int b, const uint4 (&rk)[PPT][2], const uint4 (&rv)[PPT][2]) {
+    auto stash = [&](int b, const auto &rk, const auto &rv) {
 #pragma unroll
         for (int i = 0; i < PPT; i++) {
             int pk, d0;
-            pair_of<HD>(tid + i * AT, pk, d0);
-            stage_pair<KLD>(sk[b], svt[b], pk, d0, rk[i][0], rk[i][1], rv[i][0], rv[i][1]);
+            pair_of<HD>((tid + i * NT) % UPT, pk, d0);
+            u16 *t = stg[b] + (tid + i * NT) / UPT * TS;
+            stage_pair<KLD>(t, t + BKV * KLD, pk, d0, rk[i][0], rk[i][1], rv[i][0], rv[i][1]);
         }
     };
     fetch(0, rk0, rv0);
-    fetch(1, rk1, rv1);   /* past the last tile: the last position again, unused */
+    if constexpr (NSET == 2) fetch(1, rk1, rv1);   /* past the last step: the last position again, unused */
 
     /* this wave's queries: block rows wr0 .. wr0+31; lane l takes row wr0 + l%32 */
-    const int wr0 = wave * 32;
+    const int wr0 = qg * 32;
     const bool wave_active = wr0 < nrows;
     const int wave_first = p0 + wr0, wave_last = p0 + min(wr0 + 31, nrows - 1);
     const int qrow = wr0 + (lane & 31);
@@ -269,32 +299,73 @@ __global__ void __launch_bounds__(AT) k_attn_prefill_blk(
     for (int j = 0; j < DT; j++) o[j] = (f32x16){};
     float mrow = -INFINITY, lrow = 0.f;
 
+    auto compute = [&](int st, int b) {
+        const int k0 = (st * KG + kg) * BKV;
+        const u16 *t = stg[b] + kg * TS;
+        if (wave_active && k0 <= wave_last) {     /* wave-uniform */
+            /* every key visible to every query (at hd 128 the two forms side by
+             * side spill 60 registers, the masked one alone none) */
+            if (HD == 64 && k0 + BKV - 1 <= wave_first)
+                tile_update<HD, KLD, false>(t, t + BKV * KLD, qb16, k0, qp, scale, o, mrow, lrow);
+            else
+                tile_update<HD, KLD, true>(t, t + BKV * KLD, qb16, k0, qp, scale, o, mrow, lrow);
+        }
+    };
     stash(0, rk0, rv0);
     __syncthreads();
-    /* tile kt: fetch tile kt+2 into the set tile kt left (unconditionally, so
-     * the compiler waits only for the older set), compute kt, store kt+1 */
-    auto body = [&](int kt, uint4 (&rka)[PPT][2], uint4 (&rva)[PPT][2], const uint4 (&rkb)[PPT][2],
-                    const uint4 (&rvb)[PPT][2]) {
-        const int b = kt & 1;
-        fetch(kt + 2, rka, rva);
-        const int k0 = kt * BKV;
-        if (wave_active && k0 <= wave_last) {     /* wave-uniform */
-            if (k0 + BKV - 1 <= wave_first)       /* every key visible to every query */
-                tile_update<HD, KLD, false>(sk[b], svt[b], qb16, k0, qp, scale, o, mrow, lrow);
-            else
-                tile_update<HD, KLD, true>(sk[b], svt[b], qb16, k0, qp, scale, o, mrow, lrow);
+    if constexpr (NSET == 2) {
+        /* step t: fetch step t+2 into the set step t left (unconditionally, so
+         * the compiler waits only for the older set), compute t, store t+1 */
+        auto body = [&](int st, auto &rka, auto &rva, const auto &rkb, const auto &rvb) {
+            const int b = st & 1;
+            fetch(st + 2, rka, rva);
+            compute(st, b);
+            if (st + 1 < nsteps) stash(b ^ 1, rkb, rvb);
+            __syncthreads();
+        };
+        for (int st = 0; st < nsteps; st += 2) {
+            body(st, rk0, rv0, rk1, rv1);
+            if (st + 1 < nsteps) body(st + 1, rk1, rv1, rk0, rv0);
         }
-        if (kt + 1 < ntiles) stash(b ^ 1, rkb, rvb);
+    } else {
+        for (int st = 0; st < nsteps; st++) {
+            if (st + 1 < nsteps) fetch(st + 1, rk0, rv0);
+            compute(st, st & 1);
+            if (st + 1 < nsteps) stash((st + 1) & 1, rk0, rv0);
+            __syncthreads();
+        }
+    }
+    /* finish the row sum across the lane pair: element i of o[j] is dim
+     * j*32 + 8*(i/4) + 4*g + i%4 of query l%32 */
+    float l = lrow + xor32_f(lrow);
+    if constexpr (KG == 2) {
+        /* the upper key half's (m, l, O) through LDS (every wave is past its
+         * last read of the staging area) */
+        float *mo = (float *)&stg[0][0], *mm = mo + QG * 32 * MLD, *ml = mm + QG * 32;
+        if (kg == 1) {
+            if (g == 0) {
+                mm[qrow] = mrow;
+                ml[qrow] = l;
+            }
+#pragma unroll
+            for (int j = 0; j < DT; j++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    mo[qrow * MLD + j * 32 + 8 * (i >> 2) + 4 * g + (i & 3)] = o[j][i];
+        }
         __syncthreads();
-    };
-    for (int kt = 0; kt < ntiles; kt += 2) {
-        body(kt, rk0, rv0, rk1, rv1);
-        if (kt + 1 < ntiles) body(kt + 1, rk1, rv1, rk0, rv0);
+        if (kg == 1) return;
+        const float m1 = mm[qrow], M = fmaxf(mrow, m1);   /* (this half holds key 0: m is finite) */
+        const float f0 = __builtin_amdgcn_exp2f(mrow - M);
+        const float f1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - M);
+        l = fmaf(ml[qrow], f1, l * f0);
+#pragma unroll
+        for (int j = 0; j < DT; j++)
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                o[j][i] = fmaf(mo[qrow * MLD + j * 32 + 8 * (i >> 2) + 4 * g + (i & 3)], f1, o[j][i] * f0);
     }
     if (!wave_active) return;
-    /* finish the row sum across the lane pair and write O / l:
-     * element i of o[j] is dim j*32 + 8*(i/4) + 4*g + i%4 of query l%32 */
-    const float l = lrow + xor32_f(lrow);
     if (qrow < nrows) {
         const float inv = 1.0f / l;
         u16 *op = out + (size_t)(row0 + qrow) * NQ + h * HD;
@@ -318,7 +389,7 @@ __global__ void __launch_bounds__(AT) k_attn_prefill_blk(
 template <int HD, typename KT>
 __global__ void __launch_bounds__(AT) k_attn_prefill_split(
     const float *__restrict__ q, const KT *__restrict__ kc, const KT *__restrict__ vc,
-    const int *__restrict__ pos, const int *__restrict__ slot, int S, int nqb, int H, int Hkv,
+    const int *__restrict__ pos, const int *__restrict__ slot, int S, int nseq, int nqb, int H, int Hkv,
     int max_seq, u16 *__restrict__ out)
 {
     constexpr int KLD = HD + 8;          /* K tile row stride (halves)   */
@@ -334,8 +405,8 @@ __global__ void __launch_bounds__(AT) k_attn_prefill_split(
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int seq = small_div(blockIdx.x, nqb), qb = blockIdx.x - seq * nqb;
-    const int h = blockIdx.y;
+    int h, seq, qb;
+    block_of(blockIdx.x, nqb, nseq, H, h, seq, qb);
     const int kvh = small_div(h, small_div(H, Hkv));
     const int NQ = H * HD;
     const int row0 = seq * S + qb * BQS;           /* first row of the block       */
@@ -484,10 +555,13 @@ extern "C" int lmk_last_rows(hipStream_t s, const float *x, const float *q, int 
     return hipGetLastError();
 }
 
-/* Work-group count of the 128-query kernel below which the 32-query kernel
- * is used (measured: 24 blocks of 128 (one 256-token prompt, 12 heads) run
- * 1.7x faster split; 192 (eight prompts) 1.3x faster shared). */
-#define BLK_MIN_WGS 128
+/* Work-groups of 128 queries from which the shared-tile kernel is taken.  us per
+ * launch, split / shared:
+ *   hd 64, 12 heads   1 x 1300 (132) 14.8 / 17.8   1 x 1900 (180) 24.0 / 25.8
+ *                     3 x 600 (180) 13.9 / 12.7    8 x 256 (192) 10.8 / 8.8
+ *   hd 128, 16 heads  1 x 512 (64) 12.6 / 18.6     1 x 700 (96) 19.1 / 23.2
+ *                     1 x 1900 (240) - / 53 (64 with four waves, 70 before) */
+#define BLK_MIN_WGS(hd) ((hd) == 64 ? 160 : 120)
 
 extern "C" int lmk_attn_prefill(hipStream_t s, const float *q, const void *kc, const void *vc,
                                 int kv_f32, const int *pos, const int *slot, int S, int nseq,
@@ -495,23 +569,38 @@ extern "C" int lmk_attn_prefill(hipStream_t s, const float *q, const void *kc, c
 {
     if (S < 1 || nseq < 1 || H < 1 || Hkv < 1 || H % Hkv || !pos || !slot) return hipErrorInvalidValue;
     if (hd != 64 && hd != 128) return hipErrorInvalidValue;
-    const int nqb_blk = (S + BQB - 1) / BQB;
-    if ((long)nqb_blk * nseq * H >= BLK_MIN_WGS) {
-        dim3 grid(nqb_blk * nseq, H);
-#define LAUNCH_AP(HD_, KT_)                                                                      \
-    hipLaunchKernelGGL((k_attn_prefill_blk<HD_, KT_>), grid, dim3(AT), 0, s, q, (const KT_ *)kc,  \
-                       (const KT_ *)vc, pos, slot, S, nqb_blk, H, Hkv, max_seq, out)
+    /* (block_of divides by small_div: ids below 2^20, divisors below 2^12) */
+    if ((long)((S + BQS - 1) / BQS) * nseq * H >= 1 << 20 || nseq >= 1 << 12 || H >= 1 << 12)
+        return hipErrorInvalidValue;
+    if ((long)((S + 127) / 128) * nseq * H >= BLK_MIN_WGS(hd)) {
+        /* hd 128: eight waves, two key tiles a step (two waves a SIMD); hd 64:
+         * 64-query blocks of four waves, two key tiles a step, unless the
+         * sequences are short (20 x 90 rows, 16 heads: 10.2 us against 8.8 with
+         * 128-query blocks, which then stage each tile once) */
+#define LAUNCH_APV(HD_, KT_, QG_, W_)                                                                      \
+    do {                                                                                                   \
+        const int nqb = (S + 32 * QG_ - 1) / (32 * QG_);   /* blocks of the kernel's own 32 * QG queries */ \
+        hipLaunchKernelGGL((k_attn_prefill_blk<HD_, KT_, QG_, W_>), dim3(nqb * nseq * H), dim3(64 * W_), 0, s, q, \
+                           (const KT_ *)kc, (const KT_ *)vc, pos, slot, S, nseq, nqb, H, Hkv, max_seq, out);      \
+    } while (0)
+#define LAUNCH_AP(HD_, KT_)                                      \
+    do {                                                         \
+        if constexpr (HD_ == 128) LAUNCH_APV(HD_, KT_, 4, 8);    \
+        else if (S > 128) LAUNCH_APV(HD_, KT_, 2, 4);            \
+        else LAUNCH_APV(HD_, KT_, 4, 4);                         \
+    } while (0)
         if (hd == 64 && kv_f32) LAUNCH_AP(64, float);
         else if (hd == 64) LAUNCH_AP(64, u16);
         else if (kv_f32) LAUNCH_AP(128, float);
         else LAUNCH_AP(128, u16);
 #undef LAUNCH_AP
+#undef LAUNCH_APV
     } else {
         const int nqb = (S + BQS - 1) / BQS;
-        dim3 grid(nqb * nseq, H);
+        dim3 grid(nqb * nseq * H);
 #define LAUNCH_AP(HD_, KT_)                                                                        \
     hipLaunchKernelGGL((k_attn_prefill_split<HD_, KT_>), grid, dim3(AT), 0, s, q, (const KT_ *)kc, \
-                       (const KT_ *)vc, pos, slot, S, nqb, H, Hkv, max_seq, out)
+                       (const KT_ *)vc, pos, slot, S, nseq, nqb, H, Hkv, max_seq, out)
         if (hd == 64 && kv_f32) LAUNCH_AP(64, float);
         else if (hd == 64) LAUNCH_AP(64, u16);
         else if (kv_f32) LAUNCH_AP(128, float);
