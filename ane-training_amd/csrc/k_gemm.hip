@@ -1195,9 +1195,12 @@ static void launch_tile_split(hipStream_t s, const uint16_t *A, int lda, const u
  * back to back, best of 5; the fit is within 12% where the choice lies):
  *   tile               fixed  floor  slope   per CU  waves
  *   64 x 64 (4 waves)   2.5   0.33   0.235     3      12
- *   64 x 128 (4)        2.7   0.40   0.36      2       8
+ *   64 x 128 (4)        3.5   0.40   0.36      2       8
  *   128 x 128 (8)       3.7   0.60   0.60      1       8
  *   256 x 128 (8)       5.0   1.05   1.05      1       8
+ * (64 x 128 priced 0.8 us above its plain store for its longer epilogues: the
+ * Wo + residual + norm of 2048 x 768 x 768 took 12.3 us on it against 11.5 on
+ * 64 x 64, the 8 x 256 scored forward 1229 us against 1212.)
  * Small tiles start and end sooner and quantise finer; large ones move fewer
  * operand bytes per product through L2 and LDS.  Measured (us) where 64 x 64
  * was used before, 64 x 64 / 64 x 128 / 128 x 128 / 256 x 128:
@@ -1217,7 +1220,7 @@ static int pick_tile(int M, int N, int K, bool qkv)
 {
     static const struct { int bm, bn; float fixed, floor, slope; } T[4] = {
         {64, 64, 2.5f, 0.33f, 0.235f},
-        {64, 128, 2.7f, 0.40f, 0.36f},
+        {64, 128, 3.5f, 0.40f, 0.36f},
         {128, 128, 3.7f, 0.60f, 0.60f},
         {256, 128, 5.0f, 1.05f, 1.05f}};
     int best = TILE_64x64;
