@@ -1383,18 +1383,12 @@ int lm_generate_greedy(LMModel *m, int B, const int *first_tokens, const int *po
     return check_err(m, m->h_hdr[LM_HDR_ERR]);
 }
 
-/* Causal forward of nseq sequences of S tokens (sequence i: slot slots[i],
- * positions pos0[i] .. pos0[i]+S-1, positions below pos0[i] already cached)
- * on the MFMA path, in chunks of whole sequences.  logits_mode LM_LOGITS_ALL:
- * every row's logits; LM_LOGITS_LAST: the last row of each sequence.  Host
- * `logits` (may be NULL) receives them in sequence order; the last chunk's
- * logits stay in d_logits. */
 /* The layers of a prefill chunk of R rows (sequences of S rows; tokens,
- * positions and slots, R ints each, read from h_rin into d_rin) and the classifier into d_logits,
- * of every row with `all`, else of each sequence's last row (positions and
- * slots after the rows', R/S ints each): launched directly the first
- * time a shape comes and replayed from a captured graph from its second time
- * on, unless graphs are off.  A prompt's length is often its own: prompts of 30
+ * positions and slots, R ints each, read from h_rin into d_rin) and the
+ * classifier into d_logits, of every row with `all`, else of each sequence's
+ * last row (positions and slots after the rows', R/S ints each): launched
+ * directly the first time a shape comes and replayed from a captured graph from
+ * its second time on, unless graphs are off.  A prompt's length is often its own: prompts of 30
  * to 59 tokens, each a new length, took 260 us more than a replay when each was
  * captured (707 us a call against 446), 130 launched directly (479 against 350),
  * and the captures threw out the graphs kept. */
@@ -1447,6 +1441,12 @@ static int run_rows(LMModel *m, int R, int S, int all)
     return LM_OK;
 }
 
+/* Causal forward of nseq sequences of S tokens (sequence i: slot slots[i],
+ * positions pos0[i] .. pos0[i]+S-1, positions below pos0[i] already cached)
+ * on the MFMA path, in chunks of whole sequences.  logits_mode LM_LOGITS_ALL:
+ * every row's logits; LM_LOGITS_LAST: the last row of each sequence.  Host
+ * `logits` (may be NULL) receives them in sequence order; the last chunk's
+ * logits stay in d_logits. */
 static int run_prefill(LMModel *m, int nseq, const int *slots, const int *pos0, const int *tokens,
                        int S, int logits_mode, float *logits, float *loss)
 {
