@@ -304,7 +304,9 @@ MFMA_PEAK_TFLOPS = 2500.0      # dense fp16
 def _timed(m, fn, reps):
     """Device milliseconds per call of fn over reps calls (hipEvents on the
     model's stream; fn's host copies of the results are excluded by design of
-    the calls used: they keep logits on the device)."""
+    the calls used: they keep logits on the device).  Two calls come before: a
+    prompt's shape launches directly the first time and is captured the second."""
+    fn()
     fn()
     m.sync()
     m.timer_begin()
