@@ -144,11 +144,12 @@ __device__ __forceinline__ void tile_update(const u16 *sk, const u16 *svt, const
             mx = fmaxf(mx, sacc[nt][i]);
         }
     mx = fmaxf(mx, xor32_f(mx)) * scale;
-    /* a query with every key so far masked keeps m = -inf (and O = l = 0) */
+    /* a query with every key so far masked keeps m = -inf (and O = l = 0), also
+     * where another query of the wave raises its own */
     const bool raise = mx > mrow + M_SLACK;
     if (__builtin_amdgcn_ballot_w64(raise)) {     /* wave-uniform */
         const float mn = raise ? mx : mrow;
-        const float corr = __builtin_amdgcn_exp2f(mrow - mn);   /* 0 from m = -inf, 1 if kept */
+        const float corr = raise ? __builtin_amdgcn_exp2f(mrow - mn) : 1.f;   /* 0 from m = -inf */
         lrow *= corr;
 #pragma unroll
         for (int j = 0; j < DT; j++) o[j] *= corr;

@@ -28,3 +28,24 @@ def test_blocks_match_small_pieces(lm, d, n, S, kv32):
             ref = np.concatenate([m.prefill(toks[i, p:p + 32], slot=i, pos0=p) for p in range(0, S, 32)])
             np.testing.assert_allclose(got[i], ref, rtol=1e-2, atol=2e-2)
             assert np.abs(got[i] - ref).mean() < 2e-3
+
+
+@pytest.mark.parametrize("d", [HD64, HD128], ids=["hd64", "hd128"])
+@pytest.mark.parametrize("pos0,S", [(1, 1300), (10, 1200), (40, 1200), (63, 1300), (100, 1200),
+                                    (1, 64), (10, 100), (40, 41), (63, 65), (100, 160)])
+@pytest.mark.parametrize("kv32", [False, True])
+def test_offsets_that_straddle_a_key_tile(lm, d, pos0, S, kv32):
+    """Prompts behind pos0 cached positions, pos0 no multiple of 32: a group of 32
+    queries then holds some that see none of a wave's first key tile beside
+    some that do.  The bound of the test above (pieces at multiples of 32 have
+    no such group)."""
+    cfg = lm.make_config(**d)
+    w16 = lm.synth_weights_f16(cfg, 103, 0.03, True)
+    toks = np.random.default_rng(S + pos0).integers(0, 300, pos0 + S).astype(np.int32)
+    with lm.Model.create(cfg, w16, True, 1, pos0 + S) as m:
+        m.set_option(lm.LM_OPT_KV_F32, int(kv32))
+        ref = np.concatenate([m.prefill(toks[p:p + 32], pos0=p) for p in range(0, pos0 + S, 32)])[pos0:]
+        got = m.prefill(toks[pos0:], pos0=pos0)
+    assert np.all(np.isfinite(got)), np.unique(np.argwhere(~np.isfinite(got))[:, 0])[:8]
+    np.testing.assert_allclose(got, ref, rtol=1e-2, atol=2e-2)
+    assert np.abs(got - ref).mean() < 2e-3
