@@ -26,8 +26,8 @@ def regset(tok):
     return {tok} if m else set()
 
 
-MAX_QUEUE = 64     # operations remembered per path (more than a wait can name)
-
+YOUNGEST = 64      # operations whose order is kept: a wait names at most 63 of them
+NOTHING = ((frozenset(), False), ())
 
 def blocks_of(body):
     """Basic blocks [(label, [instructions])] in text order."""
@@ -46,41 +46,44 @@ def blocks_of(body):
     return out
 
 
-def run_block(instrs, queue, report):
-    """The lgkm operations in flight after the block, oldest first: (destination
-    registers, is scalar memory).  LDS operations complete in order, so a wait
-    lgkmcnt(n) retires all but the n youngest; scalar loads complete out of
-    order, so with one in flight only lgkmcnt(0) retires anything."""
-    queue = list(queue)
+def run_block(instrs, state, report):
+    """The lgkm operations in flight after the block: ((destination registers of
+    the older ones, whether a scalar load is among them), the youngest ones in
+    order, oldest first, each (destination registers, is scalar memory)).  LDS
+    operations complete in order, so a wait lgkmcnt(n) retires all but the n
+    youngest: the order of those older than any n is not needed, only what they
+    still have to write.  Scalar loads complete out of order, so with one in
+    flight only lgkmcnt(0) retires anything."""
+    (old, old_scalar), young = state
+    young = list(young)
     for t in instrs:
         ops = [x for x in re.split(r"[ ,]+", t) if x]
-        if ops[0].startswith("ds_"):
+        lds, scalar = ops[0].startswith("ds_"), ops[0].startswith(("s_load", "s_buffer_load"))
+        if lds or scalar:
             dst = regset(ops[1]) if ops[0].startswith(("ds_read", "ds_bpermute", "ds_permute",
                                                        "ds_swizzle")) else set()
-            queue.append((frozenset(dst), False))
-            queue = queue[-MAX_QUEUE:]
-            continue
-        if ops[0].startswith(("s_load", "s_buffer_load")):
-            queue.append((frozenset(), True))
-            queue = queue[-MAX_QUEUE:]
+            young.append((frozenset(dst), scalar))
+            if len(young) > YOUNGEST:
+                d, sc = young.pop(0)
+                old, old_scalar = old | d, old_scalar or sc
             continue
         if ops[0] == "s_waitcnt":
             m = re.search(r"lgkmcnt\((\d+)\)", t)
-            if m:
-                n = int(m.group(1))
-                if n == 0:
-                    queue = []
-                elif not any(s for _, s in queue):
-                    queue = queue[-n:] if n < len(queue) else queue
+            n = int(m.group(1)) if m else YOUNGEST
+            if n == 0:
+                old, old_scalar, young = frozenset(), False, []
+            elif n < YOUNGEST and not old_scalar and not any(sc for _, sc in young):
+                old = frozenset()
+                young = young[-n:]
             continue
-        pending = set().union(*(d for d, _ in queue)) if queue else set()
+        pending = old.union(*(d for d, _ in young))
         if pending:
             used = set()
             for o in ops[1:]:
                 used |= regset(o)
             if used & pending:
                 report(t)
-    return tuple(queue)
+    return (old, old_scalar), tuple(young)
 
 
 def check(asm_text):
@@ -93,14 +96,14 @@ def check(asm_text):
         at = {lab: i for i, (lab, _) in enumerate(blocks) if lab}
         seen = [set() for _ in blocks]
         found = set()
-        work = [(0, ())]
+        work = [(0, NOTHING)]
         while work:
-            i, queue = work.pop()
-            if queue in seen[i]:
+            i, state = work.pop()
+            if state in seen[i]:
                 continue
-            seen[i].add(queue)
+            seen[i].add(state)
             instrs = blocks[i][1]
-            after = run_block(instrs, queue, lambda t, i=i: found.add((i, t)))
+            after = run_block(instrs, state, lambda t, i=i: found.add((i, t)))
             last = instrs[-1] if instrs else ""
             m = re.match(r"s_c?branch\w*\s+(\.LBB\w+)", last)
             if m:
