@@ -59,9 +59,16 @@ def run_block(instrs, state, report):
     for t in instrs:
         ops = [x for x in re.split(r"[ ,]+", t) if x]
         lds, scalar = ops[0].startswith("ds_"), ops[0].startswith(("s_load", "s_buffer_load"))
+        returns = ops[0].startswith(("ds_read", "ds_bpermute", "ds_permute", "ds_swizzle"))
+        pending = old.union(*(d for d, _ in young))
+        if pending:
+            used = set()
+            for o in ops[2 if returns else 1:]:   # (a later read of the same register lands later)
+                used |= regset(o)
+            if used & pending:
+                report(t)
         if lds or scalar:
-            dst = regset(ops[1]) if ops[0].startswith(("ds_read", "ds_bpermute", "ds_permute",
-                                                       "ds_swizzle")) else set()
+            dst = regset(ops[1]) if returns else set()
             young.append((frozenset(dst), scalar))
             if len(young) > YOUNGEST:
                 d, sc = young.pop(0)
@@ -75,14 +82,6 @@ def run_block(instrs, state, report):
             elif n < YOUNGEST and not old_scalar and not any(sc for _, sc in young):
                 old = frozenset()
                 young = young[-n:]
-            continue
-        pending = old.union(*(d for d, _ in young))
-        if pending:
-            used = set()
-            for o in ops[1:]:
-                used |= regset(o)
-            if used & pending:
-                report(t)
     return (old, old_scalar), tuple(young)
 
 

@@ -31,6 +31,13 @@ def test_flags_copy_of_pending_register():
     assert len(check_lds_asm.check(asm)[1]) == 1
 
 
+@pytest.mark.parametrize("op", ["ds_write_b32 v1, v5", "ds_write_b32 v4, v2", "ds_read_b32 v20, v6"])
+def test_flags_lds_operation_on_pending_register(op):
+    """As data, and as the address of a write or another read."""
+    asm = HEAD + f"\tds_read_b128 v[4:7], v1\n\t{op}\n\ts_waitcnt lgkmcnt(0)\n" + TAIL
+    assert len(check_lds_asm.check(asm)[1]) == 1
+
+
 def test_passes_use_after_wait_and_unrelated_work():
     asm = HEAD + ("\tds_read_b128 v[4:7], v1\n"
                   "\tv_mfma_f32_32x32x16_f16 a[16:31], v[12:15], v[8:11], a[16:31]\n"
