@@ -57,3 +57,28 @@ def test_greedy_ids_equal_single_steps(lm, B, steps):
         for t in range(steps):
             tk = m.forward_batch(tk, np.full(B, t, np.int32), want_logits=False)[1]
             assert np.array_equal(ids[t], tk), t
+
+
+@pytest.mark.parametrize("B", [1, 3, 5, 64])
+def test_first_step_equals_its_replays(lm, B):
+    """A handle's first step of a batch and kind is launched directly and captured
+    behind that launch; its second replays the capture: the same bits, also
+    with other work of the handle between them."""
+    rng = np.random.default_rng(B)
+    tk = rng.integers(0, 301, B).astype(np.int32)
+    pos = np.full(B, 2, np.int32)
+    rows = rng.integers(0, 301, (B, 2)).astype(np.int32)
+    with _model(lm, 301, B, 64) as m:
+        m.prefill_batch(rows, mode=lm.LM_LOGITS_LAST, want_logits=False)
+        first = m.forward_batch(tk, pos)
+        ids = m.forward_batch(tk, pos, want_logits=False)[1]
+        for _ in range(3):
+            lg, am = m.forward_batch(tk, pos)
+            assert np.array_equal(lg, first[0]) and np.array_equal(am, first[1])
+            assert np.array_equal(m.forward_batch(tk, pos, want_logits=False)[1], ids)
+            m.prefill_batch(rows, mode=lm.LM_LOGITS_LAST)
+        assert np.array_equal(ids, first[1])
+        runs = [m.generate_greedy(first[1], pos + 1, 37) for _ in range(3)]
+        m.set_option(lm.LM_OPT_USE_GRAPH, 0)
+        runs.append(m.generate_greedy(first[1], pos + 1, 37))
+        assert all(np.array_equal(r, runs[0]) for r in runs)
