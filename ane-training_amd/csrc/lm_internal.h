@@ -34,6 +34,23 @@ int lmh_weights_untied(const LMWeights *w);
 int lmh_read_llama2c(const char *path, Config *cfg, int *untied, float **data);
 int lmh_read_blzt(const char *path, Config *cfg, float **data);
 
+/* ---- prompt shapes kept as graphs (lm_shapes.c) ----------------------------
+ * A shape: R rows in sequences of S, all logits or the last rows'.  used: the
+ * number of the call that last had it, 0 for an empty entry. */
+#define LM_SHAPE_GRAPHS 4
+#define LM_SHAPE_SEEN 16
+typedef struct { int R, S, all; unsigned long used; } LMShape;
+typedef struct {
+    LMShape graph[LM_SHAPE_GRAPHS];   /* captured */
+    LMShape seen[LM_SHAPE_SEEN];      /* launched directly, the last ones */
+    unsigned long calls;
+} LMShapes;
+enum { LM_SHAPE_DIRECT, LM_SHAPE_CAPTURE, LM_SHAPE_REPLAY };
+
+/* What a call of this shape does: launch directly, replay graph *slot, or
+ * capture into *slot (in place of the graph that is there). */
+int lmh_shape_use(LMShapes *t, int R, int S, int all, int *slot);
+
 /* Rows of W1 and W3 are stored interleaved in blocks of LMK_GATE_BLOCK rows:
  * block j = [W1 rows j*G .. j*G+G-1, W3 rows j*G .. j*G+G-1], so any 2G-wide
  * output tile of the fused W1|W3 product holds matching h1/h3 columns. */

@@ -37,8 +37,6 @@
     } while (0)
 
 #define MAX_GEMV_B 4
-#define PREFILL_GRAPHS 4   /* prefill chunk shapes kept captured */
-#define PREFILL_SEEN 16    /* shapes remembered as launched once */
 #define GIVE_MIN_FLOATS ((size_t)1 << 20)   /* least staging of results: two 2 MiB segments */
 /* What a queued decode step takes in and gives back: a call's step with its
  * logits or with the ids alone, and the steps of a greedy run (one, or
@@ -104,17 +102,9 @@ struct LMModel {
     /* captured decode graphs by kind of step (greedy feedback stays on the
      * device) and context class: [max_batch + 1][kind][class] */
     hipGraphExec_t (*step_graph)[STEP_KINDS][CTX_CLASSES];
-    /* captured prefill chunks (the layers and, with all logits, the
-     * classifier), by rows, rows per sequence and logits mode; replaced round
-     * robin */
-    struct {
-        int R, S, all;
-        hipGraphExec_t ge;
-    } pgraph[PREFILL_GRAPHS];
-    int pgraph_next;
-    /* the last shapes launched directly: captured when they come again (run_rows) */
-    struct { int R, S, all; } pseen[PREFILL_SEEN];
-    int pseen_next;
+    /* captured prefill chunks (the layers and the classifier) of shapes.graph */
+    hipGraphExec_t pgraph[LM_SHAPE_GRAPHS];
+    LMShapes shapes;
     int use_graph;
     int ctx_cls;                /* context class of the decode step being queued */
 };
@@ -352,11 +342,11 @@ static int alloc_kv(LMModel *m)
 
 static void drop_graphs(LMModel *m)
 {
-    for (int i = 0; i < PREFILL_GRAPHS; i++)
-        if (m->pgraph[i].ge) {
-            hipGraphExecDestroy(m->pgraph[i].ge);
-            m->pgraph[i].ge = NULL;
-        }
+    for (int i = 0; i < LM_SHAPE_GRAPHS; i++) {
+        if (m->pgraph[i]) hipGraphExecDestroy(m->pgraph[i]);
+        m->pgraph[i] = NULL;
+        m->shapes.graph[i].used = 0;
+    }
     if (!m->step_graph) return;
     for (int b = 0; b <= m->max_batch; b++)
         for (int k = 0; k < STEP_KINDS * CTX_CLASSES; k++) {
@@ -1154,6 +1144,24 @@ static int enqueue_kind(LMModel *m, int B, int kind)
     return LM_OK;
 }
 
+static int capture_begin(LMModel *m)
+{
+    HIPCHK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
+    return LM_OK;
+}
+
+/* rc: the status of what was queued since capture_begin */
+static int capture_end(LMModel *m, int rc, hipGraphExec_t *ge)
+{
+    hipGraph_t g = NULL;
+    hipError_t e = hipStreamEndCapture(m->stream, &g);
+    if (rc == LM_OK && e == hipSuccess) e = hipGraphInstantiateWithFlags(ge, g, 0);
+    if (g) hipGraphDestroy(g);
+    if (rc != LM_OK) return rc;
+    HIPCHK(e);
+    return LM_OK;
+}
+
 /* Run the decode steps of `kind` of rows 0..B-1: launched directly the first
  * time, and captured while the device is busy with them, replayed from then
  * on.  Captured before its launch, a handle's first step kept the device
@@ -1169,16 +1177,8 @@ static int enqueue_decode_steps(LMModel *m, int B, int kind)
     }
     int rc = enqueue_kind(m, B, kind);
     if (rc || !m->use_graph) return rc;
-    hipGraph_t g;
-    HIPCHK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-    rc = enqueue_kind(m, B, kind);
-    hipError_t e = hipStreamEndCapture(m->stream, &g);
-    if (rc) return rc;
-    HIPCHK(e);
-    e = hipGraphInstantiateWithFlags(ge, g, 0);
-    hipGraphDestroy(g);
-    HIPCHK(e);
-    return LM_OK;
+    if ((rc = capture_begin(m))) return rc;
+    return capture_end(m, enqueue_kind(m, B, kind), ge);
 }
 
 /* Whether the decode step of B rows holds hand-off waits (the batch 1-4
@@ -1389,61 +1389,39 @@ int lm_generate_greedy(LMModel *m, int B, const int *first_tokens, const int *po
     return check_err(m, m->h_hdr[LM_HDR_ERR]);
 }
 
-/* The layers of a prefill chunk of R rows (sequences of S rows; tokens,
+/* Queue the layers of a prefill chunk of R rows (sequences of S rows; tokens,
  * positions and slots, R ints each, read from h_rin into d_rin) and the
  * classifier into d_logits, of every row with `all`, else of each sequence's
- * last row (positions and slots after the rows', R/S ints each): launched
- * directly the first time a shape comes and replayed from a captured graph from
- * its second time on, unless graphs are off.  A prompt's length is often its own: prompts of 30
- * to 59 tokens, each a new length, took 260 us more than a replay when each was
- * captured (707 us a call against 446), 130 launched directly (479 against 350),
- * and the captures threw out the graphs kept. */
-static int run_rows(LMModel *m, int R, int S, int all)
+ * last row (positions and slots after the rows', R/S ints each). */
+static int enqueue_prefill(LMModel *m, int R, int S, int all)
 {
     const int *tok = m->d_rin, *pos = m->d_rin + R, *slot = m->d_rin + 2 * (size_t)R;
     const int *lpos = all ? NULL : m->d_rin + 3 * (size_t)R, *lslot = all ? NULL : lpos + R / S;
-    const int nin = 3 * R + (all ? 0 : 2 * (R / S));
-    if (!m->use_graph || m->fold_off) {   /* (the graphs hold the folded form) */
-        KCHK(lmk_rows_in(m->stream, m->dh_rin, m->d_rin, nin));
-        return enqueue_rows(m, R, S, tok, pos, slot, m->d_logits, lpos, lslot);
-    }
+    KCHK(lmk_rows_in(m->stream, m->dh_rin, m->d_rin, 3 * R + (all ? 0 : 2 * (R / S))));
+    return enqueue_rows(m, R, S, tok, pos, slot, m->d_logits, lpos, lslot);
+}
+
+/* Run a prefill chunk: launched directly, or replayed from a captured graph of
+ * its shape, as lmh_shape_use says.  us a call, prompts of 30 to 52 tokens
+ * through Stories, 3 / 6 / 12 lengths in rotation: 301 / 307 / 311 (replays
+ * alone 301, direct launches 311); graphs replaced round robin 303 / 413 / 415. */
+static int run_rows(LMModel *m, int R, int S, int all)
+{
     int k = 0;
-    while (k < PREFILL_GRAPHS &&
-           !(m->pgraph[k].ge && m->pgraph[k].R == R && m->pgraph[k].S == S && m->pgraph[k].all == all))
-        k++;
-    if (k == PREFILL_GRAPHS) {
-        int seen = 0;
-        for (int i = 0; i < PREFILL_SEEN; i++)
-            seen |= m->pseen[i].R == R && m->pseen[i].S == S && m->pseen[i].all == all;
-        if (!seen) {
-            m->pseen[m->pseen_next].R = R;
-            m->pseen[m->pseen_next].S = S;
-            m->pseen[m->pseen_next].all = all;
-            m->pseen_next = (m->pseen_next + 1) % PREFILL_SEEN;
-            KCHK(lmk_rows_in(m->stream, m->dh_rin, m->d_rin, nin));
-            return enqueue_rows(m, R, S, tok, pos, slot, m->d_logits, lpos, lslot);
+    /* (the graphs hold the folded form) */
+    const int how = m->use_graph && !m->fold_off ? lmh_shape_use(&m->shapes, R, S, all, &k) : LM_SHAPE_DIRECT;
+    if (how == LM_SHAPE_DIRECT) return enqueue_prefill(m, R, S, all);
+    if (how == LM_SHAPE_CAPTURE) {
+        if (m->pgraph[k]) hipGraphExecDestroy(m->pgraph[k]);
+        m->pgraph[k] = NULL;
+        int rc = capture_begin(m);
+        if (rc == LM_OK) rc = capture_end(m, enqueue_prefill(m, R, S, all), &m->pgraph[k]);
+        if (rc != LM_OK) {
+            m->shapes.graph[k].used = 0;
+            return rc;
         }
-        k = m->pgraph_next;
-        m->pgraph_next = (k + 1) % PREFILL_GRAPHS;
-        if (m->pgraph[k].ge) {
-            hipGraphExecDestroy(m->pgraph[k].ge);
-            m->pgraph[k].ge = NULL;
-        }
-        hipGraph_t g;
-        HIPCHK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-        int rc = lmk_rows_in(m->stream, m->dh_rin, m->d_rin, nin) == hipSuccess ? LM_OK : LM_ERR_HIP;
-        if (rc == LM_OK) rc = enqueue_rows(m, R, S, tok, pos, slot, m->d_logits, lpos, lslot);
-        hipError_t e = hipStreamEndCapture(m->stream, &g);
-        if (rc) return rc;
-        HIPCHK(e);
-        e = hipGraphInstantiateWithFlags(&m->pgraph[k].ge, g, 0);
-        hipGraphDestroy(g);
-        HIPCHK(e);
-        m->pgraph[k].R = R;
-        m->pgraph[k].S = S;
-        m->pgraph[k].all = all;
     }
-    HIPCHK(hipGraphLaunch(m->pgraph[k].ge, m->stream));
+    HIPCHK(hipGraphLaunch(m->pgraph[k], m->stream));
     return LM_OK;
 }
 
