@@ -1402,7 +1402,9 @@ static int enqueue_prefill(LMModel *m, int R, int S, int all)
 }
 
 /* Run a prefill chunk: launched directly, or replayed from a captured graph of
- * its shape, as lmh_shape_use says.  us a call, prompts of 30 to 52 tokens
+ * its shape, as lmh_shape_use says; captured behind a direct launch, while the
+ * device is busy with it (a shape's second call 484 -> 344-499 us at 41 tokens
+ * of Stories, 1532 -> 1299 at 8 x 256).  us a call, prompts of 30 to 52 tokens
  * through Stories, 3 / 6 / 12 lengths in rotation: 301 / 307 / 311 (replays
  * alone 301, direct launches 311); graphs replaced round robin 303 / 413 / 415. */
 static int run_rows(LMModel *m, int R, int S, int all)
@@ -1410,19 +1412,17 @@ static int run_rows(LMModel *m, int R, int S, int all)
     int k = 0;
     /* (the graphs hold the folded form) */
     const int how = m->use_graph && !m->fold_off ? lmh_shape_use(&m->shapes, R, S, all, &k) : LM_SHAPE_DIRECT;
-    if (how == LM_SHAPE_DIRECT) return enqueue_prefill(m, R, S, all);
-    if (how == LM_SHAPE_CAPTURE) {
-        if (m->pgraph[k]) hipGraphExecDestroy(m->pgraph[k]);
-        m->pgraph[k] = NULL;
-        int rc = capture_begin(m);
-        if (rc == LM_OK) rc = capture_end(m, enqueue_prefill(m, R, S, all), &m->pgraph[k]);
-        if (rc != LM_OK) {
-            m->shapes.graph[k].used = 0;
-            return rc;
-        }
+    if (how == LM_SHAPE_REPLAY) {
+        HIPCHK(hipGraphLaunch(m->pgraph[k], m->stream));
+        return LM_OK;
     }
-    HIPCHK(hipGraphLaunch(m->pgraph[k], m->stream));
-    return LM_OK;
+    int rc = enqueue_prefill(m, R, S, all);
+    if (rc || how == LM_SHAPE_DIRECT) return rc;
+    if (m->pgraph[k]) hipGraphExecDestroy(m->pgraph[k]);
+    m->pgraph[k] = NULL;
+    if ((rc = capture_begin(m)) == LM_OK) rc = capture_end(m, enqueue_prefill(m, R, S, all), &m->pgraph[k]);
+    if (rc != LM_OK) m->shapes.graph[k].used = 0;
+    return rc;
 }
 
 /* Causal forward of nseq sequences of S tokens (sequence i: slot slots[i],
