@@ -82,3 +82,24 @@ def test_first_step_equals_its_replays(lm, B):
         m.set_option(lm.LM_OPT_USE_GRAPH, 0)
         runs.append(m.generate_greedy(first[1], pos + 1, 37))
         assert all(np.array_equal(r, runs[0]) for r in runs)
+
+
+@pytest.mark.parametrize("n,S", [(1, 5), (3, 33), (2, 150)])
+def test_prompt_calls_equal_their_replays(lm, n, S):
+    """A prompt shape's first call launches directly, its second captures behind
+    its launch, later ones replay: the same bits, for new tokens too, and with
+    more shapes between them than are kept."""
+    rng = np.random.default_rng(S)
+    a, b = rng.integers(0, 300, (2, n, S)).astype(np.int32)
+    with _model(lm, 300, n, 256) as m:
+        for mode in (lm.LM_LOGITS_LAST, lm.LM_LOGITS_ALL):
+            m.set_option(lm.LM_OPT_USE_GRAPH, 0)
+            want = [m.prefill_batch(t, mode=mode) for t in (a, b)]
+            m.set_option(lm.LM_OPT_USE_GRAPH, 1)
+            for k in (0, 1, 0, 1, 1, 0):
+                assert np.array_equal(m.prefill_batch((a, b)[k], mode=mode), want[k]), k
+            for L in range(2, 8):
+                for _ in range(2):
+                    m.prefill_batch(a[:, :L] if L < S else b, mode=mode)
+            for k in (0, 1, 0):
+                assert np.array_equal(m.prefill_batch((a, b)[k], mode=mode), want[k]), k
