@@ -19,9 +19,11 @@
  */
 #include "lm_internal.h"
 
+#include <limits.h>
 #include <omp.h>
 #include <pthread.h>
 #include <sched.h>
+#include <semaphore.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -43,6 +45,23 @@
  * GRAPH_STEPS), whose inputs and ids the run moves itself. */
 enum { STEP_LOGITS, STEP_IDS, STEP_GREEDY, STEP_GREEDY_N, STEP_KINDS };
 #define CTX_CLASSES 4      /* context lengths the decode attention is launched for (ctx_class) */
+
+/* A call's results on their way from the staging to the caller's memory: n
+ * floats in segments of seg, segment i through half i & 1 of the staging under
+ * number seq0 + i.  Threads t < nt take every nt'th share of each segment as it
+ * lands; prog[t]: segments that t has done.  Thread 0 is the caller; the others
+ * are the handle's own, made at its first large result: they sleep on `go`
+ * between calls. */
+#define CREW_MAX 4
+typedef struct {
+    LMModel *m;
+    float *dst;                 /* NULL: only wait */
+    size_t n, seg, nseg;
+    int seq0, nt;
+    int issued, rc, prog[CREW_MAX];
+    int hands, quit;            /* threads beside the caller's */
+    struct CrewHand { void *crew; int t; sem_t go; pthread_t id; } hand[CREW_MAX - 1];
+} Crew;
 
 struct LMModel {
     Config cfg;                 /* vocab_size positive */
@@ -105,6 +124,7 @@ struct LMModel {
     /* captured prefill chunks (the layers and the classifier) of shapes.graph */
     hipGraphExec_t pgraph[LM_SHAPE_GRAPHS];
     LMShapes shapes;
+    Crew crew;
     int use_graph;
     int ctx_cls;                /* context class of the decode step being queued */
 };
@@ -339,6 +359,8 @@ static int alloc_kv(LMModel *m)
         return LM_ERR_HIP;
     return LM_OK;
 }
+
+static void crew_end(Crew *c);
 
 static void drop_graphs(LMModel *m)
 {
@@ -696,6 +718,7 @@ void lm_free(LMModel *m)
 {
     if (!m) return;
     if (m->stream) hipStreamSynchronize(m->stream);
+    crew_end(&m->crew);
     handoff_forget(m);
     drop_graphs(m);
     free(m->step_graph);
@@ -1230,51 +1253,129 @@ static int wait_flag(LMModel *m, int set, int k, int seq)
     return LM_OK;
 }
 
-/* Copy n floats that a give kernel of `wgs` work-groups stages at src to dst
- * (NULL: only wait), share by share as they land; from 1 MiB on with up to
- * four threads (one thread copies 32 MiB to fresh pages in 1.0 ms, four in
- * 0.2-0.5, while they cross the bus in 0.58). */
-static int take(LMModel *m, int set, int seq, const float *src, float *dst, size_t n, int wgs)
+static size_t crew_len(const Crew *c, size_t i) { return (i + 1) * c->seg < c->n ? c->seg : c->n - i * c->seg; }
+
+static void crew_take(Crew *c, int t, size_t i)
 {
-    const size_t per = LM_GIVE_PER(n, wgs);
-    const int nt = dst && n >= ((size_t)1 << 18) ? (omp_get_max_threads() < 4 ? omp_get_max_threads() : 4) : 1;
-    int rc = LM_OK;
-#pragma omp parallel for num_threads(nt) schedule(static, 1) if (nt > 1)
-    for (int k = 0; k < wgs; k++) {
-        const int st = wait_flag(m, set, k, seq);
-        const size_t a = per * k, e = a + per < n ? a + per : n;
-        if (st) {
-#pragma omp atomic write
-            rc = st;
-        } else if (dst && a < e) {
-            memcpy(dst + a, src + a, (e - a) * 4);
-        }
+    const size_t len = crew_len(c, i);
+    const int wgs = give_wgs(len);
+    const size_t per = LM_GIVE_PER(len, wgs);
+    const float *src = c->m->h_logits + (i & 1) * c->seg;
+    for (int k = t; k < wgs && __atomic_load_n(&c->rc, __ATOMIC_RELAXED) == LM_OK; k += c->nt) {
+        const int st = wait_flag(c->m, (int)(i & 1), k, (int)((unsigned)c->seq0 + (unsigned)i));
+        const size_t a = per * k, e = a + per < len ? a + per : len;
+        if (st) __atomic_store_n(&c->rc, st, __ATOMIC_RELAXED);
+        else if (c->dst && a < e) memcpy(c->dst + i * c->seg + a, src + a, (e - a) * 4);
     }
-    return rc;
+    __atomic_store_n(&c->prog[t], (int)i + 1, __ATOMIC_RELEASE);
 }
 
-/* n floats of device memory (complete on the stream) to the caller's dst in
- * segments of half the staging, one crossing the bus while the host copies the
- * other; the overflow flag of the stream's work comes with them in the header. */
-static int give(LMModel *m, const float *src, float *dst, size_t n)
+/* Spin until *p >= want (0) or the crew has failed (its status). */
+static int crew_wait(Crew *c, const int *p, int want)
+{
+    for (unsigned spin = 1; __atomic_load_n(p, __ATOMIC_ACQUIRE) < want; spin++) {
+        const int rc = __atomic_load_n(&c->rc, __ATOMIC_RELAXED);
+        if (rc) return rc;
+        __builtin_ia32_pause();
+        if (!(spin & 4095)) sched_yield();
+    }
+    return LM_OK;
+}
+
+static void *crew_hand(void *arg)
+{
+    struct CrewHand *h = (struct CrewHand *)arg;
+    Crew *c = (Crew *)h->crew;
+    for (;;) {
+        while (sem_wait(&h->go) != 0) { }   /* (EINTR) */
+        if (c->quit) return NULL;
+        for (size_t i = 0; i < c->nseg && crew_wait(c, &c->issued, (int)i + 1) == LM_OK; i++)
+            crew_take(c, h->t, i);
+        __atomic_store_n(&c->prog[h->t], INT_MAX, __ATOMIC_RELEASE);   /* done with this call */
+    }
+}
+
+/* The handle's threads, as many as could be made (up to CREW_MAX - 1). */
+static int crew_hands(Crew *c)
+{
+    const int want = omp_get_max_threads() < CREW_MAX ? omp_get_max_threads() - 1 : CREW_MAX - 1;
+    while (c->hands < want) {
+        struct CrewHand *h = &c->hand[c->hands];
+        h->crew = c;
+        h->t = c->hands + 1;
+        if (sem_init(&h->go, 0, 0) != 0) break;
+        if (pthread_create(&h->id, NULL, crew_hand, h) != 0) {
+            sem_destroy(&h->go);
+            break;
+        }
+        c->hands++;
+    }
+    return c->hands < want ? c->hands : want;
+}
+
+static void crew_end(Crew *c)
+{
+    c->quit = 1;
+    for (int i = 0; i < c->hands; i++) {
+        sem_post(&c->hand[i].go);
+        pthread_join(c->hand[i].id, NULL);
+        sem_destroy(&c->hand[i].go);
+    }
+    c->hands = 0;
+}
+
+/* n floats of results to the caller's dst (NULL: only wait for them): with src,
+ * of device memory (complete on the stream), given to the staging in segments
+ * of half of it, one crossing the bus while the host copies the other; without,
+ * one segment whose give kernel is queued already under number seq0.  The
+ * header comes with them.  From 1 MiB on with up to three more threads (one
+ * thread copies 32 MiB to fresh pages in 1.0 ms, four in 0.2-0.5, while they
+ * cross the bus in 0.58), which sleep until the first share has landed. */
+static int collect(LMModel *m, const float *src, float *dst, size_t n, int seq0)
 {
     const size_t half = m->give_floats / 2 & ~(size_t)3;
-    const size_t seg = half < ((size_t)1 << 19) ? half : (size_t)1 << 19;
-    const size_t nseg = (n + seg - 1) / seg;
-    int seqs[2] = {0, 0}, rc = LM_OK;
-    for (size_t i = 0; i < nseg + 1 && rc == LM_OK; i++) {
-        if (i < nseg) {   /* segment i into half i & 1, which segment i - 2 has left */
-            const size_t a = i * seg, c = a + seg < n ? seg : n - a;
-            seqs[i & 1] = next_seq(m);
-            KCHK(lmk_give(m->stream, src + a, m->dh_logits + (i & 1) * seg, c, give_wgs(c), NULL, m->d_ovf, NULL, 0,
-                          m->dh_hdr, NULL, seqs[i & 1], m->dh_flag + (i & 1) * LM_GIVE_WGS * LM_FLAG_STRIDE));
+    Crew *c = &m->crew;
+    c->m = m;
+    c->dst = dst;
+    c->n = c->seg = n;
+    c->nseg = 1;
+    c->seq0 = seq0;
+    if (src) {
+        c->seg = half < ((size_t)1 << 19) ? half : (size_t)1 << 19;
+        c->nseg = (n + c->seg - 1) / c->seg;
+        c->seq0 = (int)((unsigned)m->seq + 1u);
+    }
+    c->nt = 1 + (dst && n >= ((size_t)1 << 18) ? crew_hands(c) : 0);
+    c->rc = LM_OK;
+    c->issued = 0;
+    for (int t = 0; t < c->nt; t++) c->prog[t] = 0;
+    int rc = LM_OK, called = 0;
+    for (size_t i = 0; i < c->nseg + 1 && rc == LM_OK; i++) {
+        if (i < c->nseg) {   /* segment i into half i & 1, which segment i - 2 has left */
+            for (int t = 1; t < c->nt && rc == LM_OK; t++) rc = crew_wait(c, &c->prog[t], (int)i - 1);
+            const size_t len = crew_len(c, i);
+            if (rc == LM_OK && src &&
+                lmk_give(m->stream, src + i * c->seg, m->dh_logits + (i & 1) * c->seg, len, give_wgs(len), NULL,
+                         m->d_ovf, NULL, 0, m->dh_hdr, NULL, next_seq(m),
+                         m->dh_flag + (i & 1) * LM_GIVE_WGS * LM_FLAG_STRIDE) != hipSuccess)
+                rc = LM_ERR_HIP;
+            if (rc == LM_OK) __atomic_store_n(&c->issued, (int)i + 1, __ATOMIC_RELEASE);
         }
-        if (i > 0) {
-            const size_t j = i - 1, a = j * seg, c = a + seg < n ? seg : n - a;
-            rc = take(m, (int)(j & 1), seqs[j & 1], m->h_logits + (j & 1) * seg, dst + a, c, give_wgs(c));
+        if (i > 0 && rc == LM_OK) {
+            if (c->nt > 1 && !called && (rc = wait_flag(m, 0, 0, c->seq0)) == LM_OK) {
+                called = 1;
+                for (int t = 1; t < c->nt; t++) sem_post(&c->hand[t - 1].go);
+            }
+            if (rc == LM_OK) {
+                crew_take(c, 0, i - 1);
+                rc = __atomic_load_n(&c->rc, __ATOMIC_RELAXED);
+            }
         }
     }
-    return rc;
+    if (rc != LM_OK) __atomic_store_n(&c->rc, rc, __ATOMIC_RELAXED);
+    for (int t = 1; called && t < c->nt; t++)
+        while (__atomic_load_n(&c->prog[t], __ATOMIC_ACQUIRE) != INT_MAX) __builtin_ia32_pause();
+    return __atomic_load_n(&c->rc, __ATOMIC_RELAXED);
 }
 
 /* The hand-off flag of the fused launches, as a call's results brought it. */
@@ -1320,7 +1421,7 @@ static int step_call(LMModel *m, const int *tokens, const int *pos, int B, int k
     __atomic_store_n(m->h_call, seq, __ATOMIC_RELEASE);
     const size_t n = kind == STEP_LOGITS ? (size_t)B * m->V : 0;
     int rc = run_decode_steps(m, B, kind, ctx_class_rows(pos, B, 0));
-    if (rc == LM_OK) rc = take(m, 0, seq, m->h_logits, logits, n, give_wgs(n));
+    if (rc == LM_OK) rc = collect(m, NULL, logits, n, seq);
     if (rc != LM_OK) {
         (void)hipStreamSynchronize(m->stream);   /* the call block is free again */
         return rc;
@@ -1380,7 +1481,7 @@ int lm_generate_greedy(LMModel *m, int B, const int *first_tokens, const int *po
         if (lmk_give_ids(m->stream, m->d_hist, m->max_seq + 1, m->d_pos, B, n_steps, t0, nt,
                          (int *)m->dh_logits, wgs, m->d_err, m->dh_hdr, seq, m->dh_flag) != hipSuccess)
             rc = LM_ERR_HIP;
-        else rc = take(m, 0, seq, m->h_logits, (float *)out_tokens + (size_t)t0 * B, (size_t)nt * B, wgs);
+        else rc = collect(m, NULL, (float *)out_tokens + (size_t)t0 * B, (size_t)nt * B, seq);
     }
     if (rc != LM_OK) {
         (void)hipStreamSynchronize(m->stream);
@@ -1498,7 +1599,7 @@ static int run_prefill(LMModel *m, int nseq, const int *slots, const int *pos0, 
             const size_t row0 = logits_mode == LM_LOGITS_ALL ? (size_t)i0 * S : (size_t)i0;
             volatile int *ovf = m->h_io + 4 * (size_t)m->max_batch + 1;
             if (rc == LM_OK && logits) {
-                rc = give(m, m->d_logits, logits + row0 * V, rows * V);
+                rc = collect(m, m->d_logits, logits + row0 * V, rows * V, 0);
                 if (rc == LM_OK) *ovf = m->h_hdr[LM_HDR_OVF];
             }
             if (rc == LM_OK && (!logits || loss) && hipStreamSynchronize(m->stream) != hipSuccess)

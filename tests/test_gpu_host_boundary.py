@@ -1,5 +1,8 @@
 """Results as kernels give them to the host (shares with a flag each, segments of
 the staging), against the device's own copy of the logits."""
+import os
+import time
+
 import numpy as np
 import pytest
 
@@ -103,3 +106,26 @@ def test_prompt_calls_equal_their_replays(lm, n, S):
                     m.prefill_batch(a[:, :L] if L < S else b, mode=mode)
             for k in (0, 1, 0):
                 assert np.array_equal(m.prefill_batch((a, b)[k], mode=mode), want[k]), k
+
+
+def test_large_results_wait_on_one_thread(lm):
+    """A call with megabytes of results waits for the device on one thread: the
+    copying threads sleep until results land, and between calls (four spinning
+    threads: four times the wall time).  They end with the handle."""
+    cfg = lm.make_config(2048, 5632, 4, 16, 8, 500, 1900)
+    w16 = lm.synth_weights_f16(cfg, 97, 0.02, True)
+    toks = np.random.default_rng(97).integers(0, 500, (1, 1900)).astype(np.int32)
+    before = None
+    for _ in range(3):
+        with lm.Model.create(cfg, w16, True, 1, 1900) as m:
+            for _ in range(3):
+                first = m.prefill_batch(toks, mode=lm.LM_LOGITS_ALL)
+            wall, cpu = time.perf_counter(), time.process_time()
+            for _ in range(15):
+                m.prefill_batch(toks, mode=lm.LM_LOGITS_ALL)
+            wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+            assert np.array_equal(m.prefill_batch(toks, mode=lm.LM_LOGITS_ALL), first)
+        assert cpu < 2.5 * wall, (cpu, wall)
+        n = len(os.listdir("/proc/self/task"))
+        assert before is None or n <= before
+        before = n
