@@ -1462,9 +1462,12 @@ __global__ void __launch_bounds__(WG) k_cls(
 /* Work-group b reduces the nblk argmax partials of row b: tok[b] = argmax
  * (lowest index on ties); with hist, also hist[b*stride + pos[b] + 1] = tok[b]
  * and pos[b] += 1 (device-resident greedy loop state).  Bound by latency: 8 KB
- * a row at 32000 columns, written a moment ago on other XCDs.  So four partials
- * a thread are in flight at once, and pos and epoch with them: classifier and
- * pick of 48 x 32000 x 768, 18.8 -> 18.1 us (one load a trip before). */
+ * a row at 32000 columns, written a moment ago on other XCDs.  So NP partials
+ * a thread are in flight at once, and pos and epoch with them: four where a
+ * thread has more than one (classifier and pick of 48 rows of 768: 32000
+ * columns 18.7 us one at a time, 18.1 four; 18000 columns 15.1 and 14.7), else
+ * one (8192 columns 12.8 one, 13.05 four with the last repeated). */
+template <int NP>
 __global__ void __launch_bounds__(WG) k_argmax_final(
     const LMArgPart *__restrict__ part, int nblk, int *__restrict__ tok, int *__restrict__ pos,
     int *__restrict__ hist, int hist_stride, unsigned *__restrict__ epoch)
@@ -1477,13 +1480,13 @@ __global__ void __launch_bounds__(WG) k_argmax_final(
     /* what the last lines need is loaded with the first partials */
     const int p = hist && threadIdx.x == 0 ? pos[b] : 0;
     const unsigned ep = epoch && b == 0 && threadIdx.x == 0 ? *epoch : 0u;
-    for (int i0 = threadIdx.x; i0 < nblk; i0 += 4 * WG) {
-        LMArgPart pt[4];
+    for (int i0 = threadIdx.x; i0 < nblk; i0 += NP * WG) {
+        LMArgPart pt[NP];
 #pragma unroll
-        for (int j = 0; j < 4; j++)   /* (past the end: the row's last again) */
-            pt[j] = part[(size_t)b * nblk + min(i0 + j * WG, nblk - 1)];
+        for (int j = 0; j < NP; j++)   /* (past the end: the row's last again) */
+            pt[j] = part[(size_t)b * nblk + (j ? min(i0 + j * WG, nblk - 1) : i0)];
 #pragma unroll
-        for (int j = 0; j < 4; j++) argmax_combine(v, id, pt[j].val, pt[j].idx);
+        for (int j = 0; j < NP; j++) argmax_combine(v, id, pt[j].val, pt[j].idx);
     }
     for (int off = 32; off > 0; off >>= 1) {
         const float ov = __shfl_xor(v, off, 64);
@@ -1796,8 +1799,10 @@ extern "C" int lmk_argmax_final(hipStream_t s, const LMArgPart *part, int nblk, 
                                 int *pos, int *hist, int hist_stride, unsigned *epoch)
 {
     if (B < 1 || nblk < 1 || !tok || (hist && !pos)) return hipErrorInvalidValue;
-    DLAUNCH(k_argmax_final, dim3(B), dim3(WG), 0, s, part, nblk, tok, pos, hist,
-                       hist_stride, epoch);
+    if (nblk > WG)
+        DLAUNCH(k_argmax_final<4>, dim3(B), dim3(WG), 0, s, part, nblk, tok, pos, hist, hist_stride, epoch);
+    else
+        DLAUNCH(k_argmax_final<1>, dim3(B), dim3(WG), 0, s, part, nblk, tok, pos, hist, hist_stride, epoch);
     return hipGetLastError();
 }
 
