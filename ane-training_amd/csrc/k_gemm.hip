@@ -28,7 +28,7 @@
  * Kernels:
  *   k_gemm_tile    work-group tile BM x BN: 64 x 64 and 64 x 128 (four waves
  *                  2 x 2), 128 x 128 and 256 x 128 (eight waves 4 x 2), the
- *                  prefill choice by pick_tile; 128 x 128 K-split in 2 for long-K
+ *                  prefill choice by lmk_pick_tile; 128 x 128 K-split in 2 for long-K
  *                  narrow GEMMs of 1024+ rows; 64 x 64 also for decode-row
  *                  classifiers, 32 x 64 for up to 32 rows (two waves), 32 x 32
  *                  (one wave) for decode-row gate GEMMs of few tiles; K streamed
@@ -1189,54 +1189,65 @@ static void launch_tile_split(hipStream_t s, const uint16_t *A, int lda, const u
 }
 
 /* Tile of a GEMM of more than 64 rows: the one with the least modelled time,
- *   fixed + stages * max(floor, slope * ceil(tiles / 256 CUs)) microseconds,
- * stages = K / 64, fitted to every tile on 19 shapes of the Stories and scaled
- * models (512-2048 rows, N 768-11264, K 768-5632; random data, 10 launches
- * back to back, best of 5; the fit is within 12% where the choice lies):
- *   tile               fixed  floor  slope   per CU  waves
- *   64 x 64 (4 waves)   2.5   0.33   0.235     3      12
- *   64 x 128 (4)        3.5   0.40   0.36      2       8
- *   128 x 128 (8)       3.7   0.60   0.60      1       8
- *   256 x 128 (8)       5.0   1.05   1.05      1       8
- * (64 x 128 priced 0.8 us above its plain store for its longer epilogues: the
- * Wo + residual + norm of 2048 x 768 x 768 took 12.3 us on it against 11.5 on
- * 64 x 64, the 8 x 256 scored forward 1229 us against 1212.)
+ *   fixed + epilogue + stages * max(floor, slope * (w + 2 ceil(w)) / 3) us,
+ * stages = K / 64, w = tiles / 256 CUs (a last round that is not full costs
+ * about two thirds of a full one), fitted to all four tiles with their real
+ * epilogues on 536 shapes (65-2048 rows, N 256-32000, K 256-5632; random data,
+ * 10 launches in a graph, best of 5):
+ *   tile               fixed  + RESNORM  GATE   QKV   floor  slope  waves per CU
+ *   64 x 64 (4 waves)   2.92     1.62    0.21   1.60  0.268  0.236      12
+ *   64 x 128 (4)        3.50     1.38    0.33    -    0.419  0.384       8
+ *   128 x 128 (8)       3.37     2.14    0.54   3.24    -    0.675       8
+ *   256 x 128 (8)       2.56    -0.03   -0.20   3.67    -    1.251       8
  * Small tiles start and end sooner and quantise finer; large ones move fewer
- * operand bytes per product through L2 and LDS.  Measured (us) where 64 x 64
- * was used before, 64 x 64 / 64 x 128 / 128 x 128 / 256 x 128:
- *   1900 x 2048 x 5632   94.8 / 60.5 / 56.2 / 80.3
- *   1900 x 2048 x 2048   31.6 / 24.0 / 22.8 / 33.2
- *   1900 x 4096 x 2048   60.6 / 45.2 / 42.6 / 39.8
- *   1024 x 2048 x 2048   16.2 / 15.2 / 18.6 / 29.6
- *   512 x 11264 x 2048   38.3 / 34.5 / 36.8 / 34.5
- *   2048 x 2304 x 768    16.0 / 17.0 / 18.0 / 16.9
- *   2048 x 768 x 768      7.3 /  7.5 /  8.9 / 13.9
- * A 1900-token prompt through four layers of the 2048-wide GQA model: 1605 ->
- * 1289 us, the same logits bit for bit.  The QKV epilogue is not built for
- * 64 x 128. */
+ * operand bytes per product through L2 and LDS.  (The 64 x 64 slope is 2% above
+ * its fit of 0.231: inside a forward the operands are colder, and ties went to
+ * the large tiles: 3 x 400 rows of the scaled GQA model 905 us, 925 with the
+ * fit's own.)  On those shapes the choice takes 0.07% longer than the best
+ * tile on average and 5.4% at most; priced by plain stores and whole rounds it
+ * took 0.45% and up to 17%, 64 x 64 below 240 tiles of 256 x 128 and those
+ * from there 2.9% and up to 84%.  Measured (us),
+ * 64 x 64 / 64 x 128 / 128 x 128 / 256 x 128, where the choice lies:
+ *   QKV      1118 x 2048 x 1024   14.4 /  -   / 15.1 / 22.6
+ *            2048 x 2304 x 768    19.9 /  -   / 24.4 / 21.9
+ *            1900 x 4096 x 2048   68.3 /  -   / 48.2 / 43.1
+ *   RESNORM  1118 x 1024 x 1024   10.7 / 11.8 / 13.7 / 22.1
+ *            2048 x 768 x 768     10.9 / 11.2 / 12.6 / 20.4
+ *            1024 x 2048 x 2048   19.0 / 18.6 / 21.4 / 35.2
+ *            1900 x 2048 x 2048   37.3 / 28.2 / 25.7 / 37.0
+ *            1900 x 2048 x 5632   99.9 / 64.6 / 56.4 / 81.3
+ *   GATE     320 x 11264 x 2048   30.1 / 24.6 / 38.8 / 35.5
+ *            1024 x 11264 x 2048  76.3 / 66.3 / 62.0 / 67.3
+ *            2048 x 4096 x 768    24.7 / 22.5 / 20.8 / 19.1
+ * The QKV epilogue is not built for 64 x 128.  The tiles give the same bits. */
 enum { TILE_64x64, TILE_64x128, TILE_128x128, TILE_256x128 };
 
-static int pick_tile(int M, int N, int K, bool qkv)
+extern "C" int lmk_pick_tile(int M, int N, int K, int epi)
 {
-    static const struct { int bm, bn; float fixed, floor, slope; } T[4] = {
-        {64, 64, 2.5f, 0.33f, 0.235f},
-        {64, 128, 3.5f, 0.40f, 0.36f},
-        {128, 128, 3.7f, 0.60f, 0.60f},
-        {256, 128, 5.0f, 1.05f, 1.05f}};
+    static const struct { int bm, bn; float fixed, resnorm, gate, qkv, floor, slope; } T[4] = {
+        {64, 64, 2.92f, 1.62f, 0.21f, 1.60f, 0.268f, 0.236f},
+        {64, 128, 3.50f, 1.38f, 0.33f, 0.f, 0.419f, 0.384f},
+        {128, 128, 3.37f, 2.14f, 0.54f, 3.24f, 0.f, 0.675f},
+        {256, 128, 2.56f, -0.03f, -0.20f, 3.67f, 0.f, 1.251f}};
     int best = TILE_64x64;
     float tb = 0.f;
     for (int i = TILE_64x64; i <= TILE_256x128; i++) {
-        if (i == TILE_64x128 && qkv) continue;
+        if (i == TILE_64x128 && epi == EPI_QKV) continue;
         const long tiles = (long)((M + T[i].bm - 1) / T[i].bm) * ((N + T[i].bn - 1) / T[i].bn);
-        const float per = T[i].slope * (float)((tiles + 255) / 256);
-        const float t = T[i].fixed + (float)(K / BKH) * (per > T[i].floor ? per : T[i].floor);
+        const float rounds = (float)tiles / 256.f + 2.f * (float)((tiles + 255) / 256);
+        const float per = T[i].slope * rounds / 3.f;
+        const float ep = epi == EPI_RESNORM || epi == EPI_RESID ? T[i].resnorm
+                         : epi == EPI_GATE                      ? T[i].gate
+                         : epi == EPI_QKV                       ? T[i].qkv
+                                                                : 0.f;
+        const float t = T[i].fixed + ep + (float)(K / BKH) * (per > T[i].floor ? per : T[i].floor);
         if (i == TILE_64x64 || t < tb) { best = i; tb = t; }
     }
     return best;
 }
 
 /* Tile choice (measured on MI355X over the Stories and scaled-model shapes):
- * more than 64 rows follow pick_tile.  Up to 64 rows take 64 x 64 tiles,
+ * more than 64 rows follow lmk_pick_tile.  Up to 64 rows take 64 x 64 tiles,
  * except: a decode-row classifier (N >= 16384, which cannot be K-split
  * ahead of its argmax) takes 64 x 64 tiles, twice the work-groups of 64 x 128
  * (C2 0.4480 -> 0.4434, C4 1.148 -> 1.142 ms/step; 32 x 64 lost at C2);
@@ -1281,7 +1292,7 @@ static int launch_gemm(hipStream_t s, const uint16_t *A, int lda, const uint16_t
         } else launch_tile<64, 64, E>(s, A, lda, W, M, N, K, e);
         return hipGetLastError();
     }
-    switch (pick_tile(M, N, K, E == EPI_QKV)) {
+    switch (lmk_pick_tile(M, N, K, E)) {
     case TILE_256x128: launch_tile<256, 128, E, RS>(s, A, lda, W, M, N, K, e); break;
     case TILE_128x128: launch_tile<128, 128, E, RS>(s, A, lda, W, M, N, K, e); break;
     case TILE_64x128:

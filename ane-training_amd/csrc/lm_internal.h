@@ -242,6 +242,9 @@ typedef struct {
 int lmk_gemm(hipStream_t s, const uint16_t *A, int lda, const uint16_t *W, int M, int N,
              int K, int epi, const LMEpilogue *ep);
 
+/* Its tile for M > 64 rows: 0 64 x 64, 1 64 x 128, 2 128 x 128, 3 256 x 128. */
+int lmk_pick_tile(int M, int N, int K, int epi);
+
 
 /* Decode rows after a K-split QKV GEMM: attention of head h, row b with q, k,
  * v summed from the ns partials part[s][b][..] (sstride floats apart) and
