@@ -556,13 +556,36 @@ extern "C" int lmk_last_rows(hipStream_t s, const float *x, const float *q, int 
     return hipGetLastError();
 }
 
-/* Work-groups of 128 queries from which the shared-tile kernel is taken.  us per
- * launch, split / shared:
- *   hd 64, 12 heads   1 x 1300 (132) 14.8 / 17.8   1 x 1900 (180) 24.0 / 25.8
- *                     3 x 600 (180) 13.9 / 12.7    8 x 256 (192) 10.8 / 8.8
- *   hd 128, 16 heads  1 x 512 (64) 12.6 / 18.6     1 x 700 (96) 19.1 / 23.2
- *                     1 x 1900 (240) - / 53 (64 with four waves, 70 before) */
-#define BLK_MIN_WGS(hd) ((hd) == 64 ? 160 : 120)
+/* Whether the 32-query kernel (split) is taken rather than the shared-tile one:
+ * up to a number of its work-groups, nseq * H * ceil(S / 32).  All of them run at
+ * once up to 512 at hd 64 (two a CU) and 256 at hd 128 (one), each a quarter of
+ * its block's tiles long; beyond that they queue, and the shared kernel stages a
+ * tile once for more queries, but its last block walks half of its sequence's
+ * tiles in turn, so that long sequences stay with the split kernel longer.
+ * Sequences of up to 64 rows end in one tile: the other waves would idle.  us
+ * per launch, split / shared (work-groups):
+ *   hd 64     1 x 1300, 12 heads (492) 14.2 / 17.6    1 x 1900 (720) 22.0 / 23.9
+ *             1 x 1500, 16 heads (752) 20.1 / 20.0    1 x 1900 (960) 25.9 / 24.1
+ *             2 x 559 (576) 10.5 / 10.7               2 x 639 (640) 12.2 / 11.1
+ *             3 x 400, 12 heads (468) 7.7 / 8.4       3 x 600 (684) 13.0 / 11.4
+ *             8 x 128, 16 heads (512) 6.0 / 6.5       10 x 128 (640) 8.5 / 6.6
+ *             16 x 64, 12 heads (384) 5.5 / 4.8       8 x 64 (192) 4.8 / 4.6
+ *   fp32      2 x 559 (576) 11.8 / 12.9               2 x 639 (640) 13.6 / 13.3
+ *             1 x 1900 (960) 32.3 / 30.2              3 x 400 (624) 12.7 / 10.8
+ *   hd 128    1 x 640 (320) 14.9 / 20.3               1 x 1000 (512) 24.1 / 26.9
+ *   16 heads  1 x 1152 (576) 32.2 / 29.7              1 x 1900 (960) 63.6 / 44.6
+ *             2 x 384 (384) 14.9 / 15.7               2 x 450 (480) 17.7 / 16.2
+ *             4 x 128 (256) 7.8 / 10.7                6 x 128 (384) 13.5 / 10.9
+ *   fp32      1 x 512 (256) 17.2 / 20.0               1 x 600 (304) 22.6 / 21.7
+ *             2 x 384 (384) 20.6 / 17.5               8 x 64 (256) 10.4 / 8.3 */
+extern "C" int lmk_attn_takes_split(int hd, int kv_f32, int H, int nseq, int S)
+{
+    const int one = hd == 64 ? 512 : 256;
+    const long wgs = (long)((S + BQS - 1) / BQS) * nseq * H;
+    if (S <= 64) return wgs <= one / 2;
+    if (S <= 256 || (hd == 128 && kv_f32)) return wgs <= one;
+    return wgs <= (hd == 64 ? one + 11 * (S - 256) / 50 : 290 + 63 * S / 256);
+}
 
 extern "C" int lmk_attn_prefill(hipStream_t s, const float *q, const void *kc, const void *vc,
                                 int kv_f32, const int *pos, const int *slot, int S, int nseq,
@@ -573,7 +596,7 @@ extern "C" int lmk_attn_prefill(hipStream_t s, const float *q, const void *kc, c
     /* (block_of divides by small_div: ids below 2^20, divisors below 2^12) */
     if ((long)((S + BQS - 1) / BQS) * nseq * H >= 1 << 20 || nseq >= 1 << 12 || H >= 1 << 12)
         return hipErrorInvalidValue;
-    if ((long)((S + 127) / 128) * nseq * H >= BLK_MIN_WGS(hd)) {
+    if (!lmk_attn_takes_split(hd, kv_f32, H, nseq, S)) {
         /* hd 128: eight waves, two key tiles a step (two waves a SIMD); hd 64:
          * 64-query blocks of four waves, two key tiles a step, unless the
          * sequences are short (20 x 90 rows, 16 heads: 10.2 us against 8.8 with

@@ -191,6 +191,10 @@ int lmk_attn_prefill(hipStream_t s, const float *q, const void *kc, const void *
                      int kv_f32, const int *pos, const int *slot, int S, int nseq,
                      int H, int Hkv, int hd, int max_seq, uint16_t *out);
 
+/* Which of its two kernels runs (1: 32-query blocks, key tiles split over the
+ * waves). */
+int lmk_attn_takes_split(int hd, int kv_f32, int H, int nseq, int S);
+
 /* The last row of each of n sequences of S rows: xo[i] = x[i*S + S-1] (D
  * floats), qo[i] = q[i*S + S-1] (NQ floats).  D and NQ multiples of 4. */
 int lmk_last_rows(hipStream_t s, const float *x, const float *q, int D, int NQ, int S, int n,

@@ -32,6 +32,7 @@ def test_blocks_match_small_pieces(lm, d, n, S, kv32):
 
 @pytest.mark.parametrize("d", [HD64, HD128], ids=["hd64", "hd128"])
 @pytest.mark.parametrize("pos0,S", [(1, 1300), (10, 1200), (40, 1200), (63, 1300), (100, 1200),
+                                    (1, 1900), (40, 1850), (63, 1937),
                                     (1, 64), (10, 100), (40, 41), (63, 65), (100, 160)])
 @pytest.mark.parametrize("kv32", [False, True])
 def test_offsets_that_straddle_a_key_tile(lm, d, pos0, S, kv32):
