@@ -55,3 +55,28 @@ def test_greedy_run_across_split_changes(lm):
                                     for p in (490, 1010)]))
     assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
     m.close()
+
+
+@pytest.mark.parametrize("d", [HD64, HD128], ids=["hd64", "hd128"])
+@pytest.mark.parametrize("B,level", [(1, 3), (1, 2), (3, 2)])
+def test_abort_ends_split_heads(lm, d, B, level):
+    """The give-up flag raised from the host before a call whose heads are split:
+    the work-groups that merge end their waits at once, the call and a greedy
+    run report LM_ERR_HIP, and the calls after them give the bits of before."""
+    m, toks = _model(lm, d, B, True)
+    m.set_option(lm.LM_OPT_FUSE_QKV_ATTN, level)
+    for p in (600, 1100, 4600):
+        pos = np.array([p, max(p - 700, 3), 40][:B], np.int32)
+        tk = toks[np.arange(B), pos]
+        want = m.forward_batch(tk, pos)[0]
+        m.set_option(lm.LM_OPT_HANDOFF_ABORT, 1)
+        with pytest.raises(lm.LMError) as ei:
+            m.forward_batch(tk, pos)
+        assert ei.value.status == lm.LM_ERR_HIP
+        assert np.array_equal(m.forward_batch(tk, pos)[0], want)
+        m.set_option(lm.LM_OPT_HANDOFF_ABORT, 1)
+        with pytest.raises(lm.LMError) as ei:
+            m.generate_greedy(tk, pos, 18)
+        assert ei.value.status == lm.LM_ERR_HIP
+        assert np.array_equal(m.forward_batch(tk, pos)[0], want)
+    m.close()
