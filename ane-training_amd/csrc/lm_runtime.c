@@ -833,7 +833,9 @@ static int chain_level(const LMModel *m, int B)
  * 512: with two, the whole-layer launch of Stories measured 12.6 against 12.1
  * us at 350 positions and 12.6 against 12.8 at 500 (the merge costs one more
  * hand-off), while 1900 positions took 23.6 us unsplit and 14.3 split over 8.
- * The class is fixed when a graph is captured, so each has its own graph. */
+ * The class is fixed when a graph is captured, so each has its own graph; where
+ * no form of the chain splits (levels 0 and 1, the whole-layer launch of more
+ * rows than one, the MFMA path) every length is class 0. */
 static int ctx_class(int p)
 {
     int c = 0;
@@ -841,10 +843,11 @@ static int ctx_class(int p)
     return c;
 }
 
-static int ctx_class_rows(const int *pos, int B, int more)
+static int ctx_class_rows(const LMModel *m, const int *pos, int B, int more)
 {
     int p = 0;
-    if (B > MAX_GEMV_B) return 0;   /* (the MFMA path has one form) */
+    const int lvl = B <= MAX_GEMV_B ? chain_level(m, B) : 0;
+    if (lvl < 2 || (lvl > 2 && B > 1)) return 0;
     for (int b = 0; b < B; b++)
         if (pos[b] > p) p = pos[b];
     return ctx_class(p + more);
@@ -1420,7 +1423,7 @@ static int step_call(LMModel *m, const int *tokens, const int *pos, int B, int k
     const int seq = next_seq(m);
     __atomic_store_n(m->h_call, seq, __ATOMIC_RELEASE);
     const size_t n = kind == STEP_LOGITS ? (size_t)B * m->V : 0;
-    int rc = run_decode_steps(m, B, kind, ctx_class_rows(pos, B, 0));
+    int rc = run_decode_steps(m, B, kind, ctx_class_rows(m, pos, B, 0));
     if (rc == LM_OK) rc = collect(m, NULL, logits, n, seq);
     if (rc != LM_OK) {
         (void)hipStreamSynchronize(m->stream);   /* the call block is free again */
@@ -1471,9 +1474,9 @@ int lm_generate_greedy(LMModel *m, int B, const int *first_tokens, const int *po
     KCHK(lmk_step_in(m->stream, m->dh_call, m->d_seq, m->d_tok, m->d_pos, B));
     int t = 0;
     for (; t + GRAPH_STEPS <= n_steps && rc == LM_OK; t += GRAPH_STEPS)
-        rc = run_decode_steps(m, B, STEP_GREEDY_N, ctx_class_rows(pos0, B, t + GRAPH_STEPS - 1));
+        rc = run_decode_steps(m, B, STEP_GREEDY_N, ctx_class_rows(m, pos0, B, t + GRAPH_STEPS - 1));
     for (; t < n_steps && rc == LM_OK; t++)
-        rc = run_decode_steps(m, B, STEP_GREEDY, ctx_class_rows(pos0, B, t));
+        rc = run_decode_steps(m, B, STEP_GREEDY, ctx_class_rows(m, pos0, B, t));
     /* the ids, as many steps at a time as the staging holds */
     const int seg = m->give_floats / B < (size_t)n_steps ? (int)(m->give_floats / B) : n_steps;
     for (int t0 = 0; t0 < n_steps && rc == LM_OK; t0 += seg) {
@@ -1732,7 +1735,7 @@ int lm_profile_chain(LMModel *m, int B, const int *tokens, const int *pos, int s
     for (int b = 0; b < B; b++)
         if (pos[b] + steps + 1 > m->max_seq) return LM_ERR_RANGE;
     const int lvl = chain_level(m, B), waits = step_waits(m, B);
-    m->ctx_cls = ctx_class_rows(pos, B, steps);
+    m->ctx_cls = ctx_class_rows(m, pos, B, steps);
     /* the launches of one step, in order: (family, layer) */
     const int nmax = 5 * m->L + 2;
     int *kf = (int *)calloc((size_t)nmax, sizeof(int)), *kl = (int *)calloc((size_t)nmax, sizeof(int));
