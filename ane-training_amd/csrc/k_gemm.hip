@@ -1152,10 +1152,11 @@ static void launch_tile(hipStream_t s, const uint16_t *A, int lda, const uint16_
         hipLaunchKernelGGL((k_gemm_tile<BM, BN, E, 3, 2, RS>), dim3(tm * tn), dim3(GT), 0, s, (const u16 *)A,
                            lda, (const u16 *)W, K, K, e, tm, tn);
     } else {
-        if (M <= 64 && BM == 64)
-            hipLaunchKernelGGL((k_gemm_tile<BM, BN, E, ring_depth<BM, BN>(true), 2, RS>), dim3(tm * tn),
-                               dim3(GT), 0, s, (const u16 *)A, lda, (const u16 *)W, K, K, e, tm, tn);
-        else if ((E == EPI_GATE || E == EPI_QKV) && !RS && BM == 64 && BN == 64 && tm * tn <= 256 &&
+        if (!RS && M <= 64 && BM == 64) {
+            if constexpr (!RS && BM == 64)
+                hipLaunchKernelGGL((k_gemm_tile<BM, BN, E, ring_depth<BM, BN>(true), 2>), dim3(tm * tn),
+                                   dim3(GT), 0, s, (const u16 *)A, lda, (const u16 *)W, K, K, e, tm, tn);
+        } else if ((E == EPI_GATE || E == EPI_QKV) && !RS && BM == 64 && BN == 64 && tm * tn <= 256 &&
                  K % (2 * BKH) == 0) {
             /* prefill-row gate or QKV, one round of tiles: K in two wave
              * groups (eight waves, two per SIMD) */
@@ -1280,7 +1281,7 @@ static int launch_gemm(hipStream_t s, const uint16_t *A, int lda, const uint16_t
     if (K % BKH) return hipErrorInvalidValue;
     if (M <= 64) {
         if constexpr (RS) {
-            launch_tile<64, 64, E, true>(s, A, lda, W, M, N, K, e);
+            return hipErrorInvalidValue;   /* (the row scale is for prefill rows) */
         } else if (N >= 16384) {
             /* decode-row classifiers (and any other wide decode-row GEMM, the
              * QKV epilogue included) on 64 x 64 tiles */
