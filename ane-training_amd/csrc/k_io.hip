@@ -49,7 +49,7 @@ __device__ __forceinline__ void raise_flag(int *flags, int seq)
 }
 
 /* n floats (src 16-byte aligned, or NULL with n 0) to dst, work-group w the
- * elements lm_give_chunk names; work-group 0 also the hand-off flag, the
+ * elements [w, w + 1) * LM_GIVE_PER(n, work-groups); work-group 0 also the hand-off flag, the
  * prefill overflow flag and B ids to the header. */
 __global__ void __launch_bounds__(IT) k_give(const float *__restrict__ src, float *__restrict__ dst, size_t n,
                                             const int *__restrict__ err, const int *__restrict__ ovf,
@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(IT) k_give(const float *__restrict__ src, floa
 
 /* The ids of steps t0 .. t0+nt-1 of an n-step greedy run of B rows that has
  * ended (pos advanced by n): out[(t - t0)*B + b]; work-group w the elements
- * lm_give_chunk names of nt*B. */
+ * [w, w + 1) * LM_GIVE_PER of nt*B. */
 __global__ void __launch_bounds__(IT) k_give_ids(const int *__restrict__ hist, int stride,
                                                 const int *__restrict__ pos, int B, int n, int t0, int nt,
                                                 int *__restrict__ out, const int *__restrict__ err,

@@ -280,8 +280,9 @@ int lmk_rownorm(hipStream_t s, float *x, int D, int M, const uint16_t *emb, cons
                 const float *sp, int ns, size_t sstride, const float *gain, uint16_t *xn);
 
 /* ---- projections of up to 64 rows (k_rows.hip) ------------------------------
- * Each with its norm, rotation, residual or gate in one launch; M <= 64, D one
- * of the model widths, K also 5632 for lmk_rows_res. */
+ * Each with its norm, rotation, residual or gate in one launch; M <= 64; D of
+ * lmk_rows_qkv and lmk_rows_gate and K of lmk_rows_res 256, 512, 768 or 1024, K
+ * also 2048 (others: hipErrorInvalidValue). */
 
 /* Rows m < M: xn = rmsnorm(x[m]) * gain, with emb of the embedding row
  * emb[tok[m]], which x[m] is set to; [Wq; Wk; Wv] xn, q and k RoPE'd at pos[m];

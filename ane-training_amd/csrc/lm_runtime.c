@@ -89,9 +89,12 @@ struct LMModel {
     uint16_t *d_xn16, *d_a16;   /* normalised rows / attention rows in fp16    */
     LMArgPart *d_amax;
     int *d_rin;                 /* prefill rows of a chunk of R: tokens, positions, slots
-                                 * (R ints each, back to back), copied in one piece;
-                                 * then R floats of loss terms (lm_prefill_loss)     */
-    int *h_rin;                 /* their pinned host staging (same layout)          */
+                                 * (R ints each, back to back), then, for the last rows'
+                                 * logits, the sequences' last positions and slots
+                                 * (k_rows_in reads them from h_rin)                 */
+    int *h_rin;                 /* their pinned host staging (same layout); with all
+                                 * logits the device writes R floats of loss terms
+                                 * after the slots (lm_prefill_loss)                 */
     int *dh_rin;                /* its device address                               */
     /* per-slot greedy state */
     int *d_tok, *d_pos, *d_hist, *d_slot_id;
@@ -423,7 +426,7 @@ static int alloc_rows(LMModel *m, int R)
         if ((st = dev_alloc((void **)&m->d_part, n * 4))) return st;
     }
     if ((st = dev_alloc((void **)&m->d_amax, r * m->cls_nblk * sizeof(LMArgPart)))) return st;
-    /* tokens, positions and slots of a chunk's rows, then its rows' loss terms */
+    /* tokens, positions and slots of a chunk's rows, then up to as many ints more */
     if ((st = dev_alloc((void **)&m->d_rin, 4 * r * 4))) return st;
     if ((st = host_alloc((void **)&m->h_rin, (void **)&m->dh_rin, 4 * r * 4))) return st;
     m->max_rows = R;
