@@ -1524,11 +1524,12 @@ static int run_rows(LMModel *m, int R, int S, int all)
         return LM_OK;
     }
     int rc = enqueue_prefill(m, R, S, all);
-    if (rc || how == LM_SHAPE_DIRECT) return rc;
+    if (how == LM_SHAPE_DIRECT) return rc;
     if (m->pgraph[k]) hipGraphExecDestroy(m->pgraph[k]);
     m->pgraph[k] = NULL;
-    if ((rc = capture_begin(m)) == LM_OK) rc = capture_end(m, enqueue_prefill(m, R, S, all), &m->pgraph[k]);
-    if (rc != LM_OK) m->shapes.graph[k].used = 0;
+    if (rc == LM_OK) rc = capture_begin(m);
+    if (rc == LM_OK) rc = capture_end(m, enqueue_prefill(m, R, S, all), &m->pgraph[k]);
+    if (rc != LM_OK) m->shapes.graph[k].used = 0;   /* (the entry is this shape's already) */
     return rc;
 }
 
