@@ -7,7 +7,9 @@
  * opaque handle, NULL on failed creation with a status code, negative int
  * status on failure, caller-owned host buffers, a message on stderr for every
  * failure.  A handle is single-threaded and not re-entrant; distinct handles
- * may be used from distinct threads.
+ * may be used from distinct threads.  From its first result of 1 MiB on, a
+ * handle keeps up to three threads of its own that help copy such results out;
+ * they sleep between calls and end with lm_free.
  *
  * Reference interfaces replaced (paths relative to the reference repository):
  *   Config                  training/model.h:19-21 (= Llama2Config,
